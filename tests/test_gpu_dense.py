@@ -66,3 +66,21 @@ def test_every_doc_and_errors(rt):
         assert [x[0] for x in got] == [ids[p] for p in pos]
     with pytest.raises(MantaRocmError, match="topk limit 0 out of range"):
         rt.dense_topk(index.rows, rt.to_device(q), 0)
+
+
+@pytest.mark.parametrize("n,d,nq,f16", [
+    # row tiles of 128 / 256 and query tiles of 4 / 8 / 16 / 32 / 64, at their
+    # edges; lengths below, at and past a stage of 32 elements, with and
+    # without whole 16-byte groups
+    (1, 1, 1, False), (255, 31, 3, False), (257, 33, 5, True), (65537, 32, 8, True), (65600, 65, 9, False),
+    (33000, 40, 17, False), (32769, 36, 33, False), (16400, 28, 65, False), (16385, 56, 130, True)])
+def test_dense_scores_tile_edges(rt, n, d, nq, f16):
+    """The score matrix equals dotRows bit for bit (one f32 chain per pair)."""
+    q = synth.normal_f32(44, 1, nq, d, 1.0)
+    if f16:
+        rows = synth.normal_f16(44, 0, n, d, 1.0)
+        docs = orc.f16_to_f32(rows)
+    else:
+        rows = docs = synth.normal_f32(44, 0, n, d, 1.0)
+    got = rt.dense_scores(rt.to_device(rows), rt.to_device(q)).download()
+    np.testing.assert_array_equal(got, orc.dot_rows(q, docs))
