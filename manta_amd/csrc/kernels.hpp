@@ -335,6 +335,12 @@ hipError_t launch_enc_add_layernorm(const float* a, const float* b, float* y, in
 hipError_t launch_enc_to_f16(const float* x, int64_t n, uint16_t* out, hipStream_t s);
 hipError_t launch_enc_gelu(float* x, int64_t n, hipStream_t s);
 
+// Whole top-k of each score row in one launch (k <= 192 and few enough parts):
+// parts per row, 0 when the shape takes the two launches below; partial
+// [rows][parts][k], tickets [rows] zero between calls.
+int64_t topk_rows_parts(int64_t rows, int64_t cols, int64_t k);
+hipError_t launch_topk_rows(const float* scores, int64_t rows, int64_t cols, int k, int smallest, uint64_t* partial,
+                            uint32_t* tickets, int32_t* ids, float* values, hipStream_t s);
 hipError_t launch_topk_rows_partial(const float* scores, int64_t rows, int64_t cols, int64_t seg,
                                     int parts, int k, int cap, int smallest, uint64_t* partial,
                                     hipStream_t s);

@@ -1472,6 +1472,14 @@ int manta_rocm_topk(MantaRocm* rt, const float* scores, int64_t rows, int64_t co
                     (long long)k, (long long)kMaxDeviceK);
     if (rows > 65535) return fail(err, MANTA_ROCM_UNSUPPORTED, "more than 65535 score rows");
     if (!out_ids) return fail(err, MANTA_ROCM_ERROR, "nil topk output");
+    if (const int64_t parts1 = manta::topk_rows_parts(rows, cols, k)) {
+        int rc1 = ensure_workspace(rt, (size_t)rows * parts1 * k * 8 + 256, err);
+        if (rc1) return rc1;
+        LAUNCH_TRY(manta::launch_topk_rows(scores, rows, cols, (int)k, order == MANTA_ROCM_SMALLEST,
+                                           (uint64_t*)rt->ws, rt->tickets, out_ids, out_values, rt->stream),
+                   "topk");
+        return MANTA_ROCM_OK;
+    }
     const int64_t tiles = (cols + 255) / 256;
     int64_t want_parts = std::max<int64_t>(1, 1024 / rows);
     int64_t rounds = std::max<int64_t>(1, (tiles + want_parts - 1) / want_parts);
