@@ -276,8 +276,6 @@ struct EmbedArgs {
     unsigned long long* err;    // first out-of-range gather index
     unsigned int* tickets;      // [batches] zero between calls (single-pass pooled kernel)
     uint16_t* out;              // f16 [batches][N] embeddings (single-pass pooled kernel)
-    uint16_t* Y16;              // plain matmul of embed_gemm2: f16 [M][N] output instead of Y (or nullptr)
-    int gelu;                   // with Y16: geluTensor (tanh in f32) applied to each value before the f16 rounding
 };
 
 hipError_t launch_embed_gemm(const EmbedArgs& a, bool gather, bool q8b, bool pool, hipStream_t s);
@@ -341,6 +339,50 @@ hipError_t launch_enc_gelu(float* x, int64_t n, hipStream_t s);
 int64_t topk_rows_parts(int64_t rows, int64_t cols, int64_t k);
 hipError_t launch_topk_rows(const float* scores, int64_t rows, int64_t cols, int k, int smallest, uint64_t* partial,
                             uint32_t* tickets, int32_t* ids, float* values, hipStream_t s);
+// encoder with f16 weight products (kernels_enc16.hip; d and h multiples of 128)
+struct EncPrepArgs {
+    const int8_t* codes[6];     // [K][N]
+    uint16_t* wt[6];            // f16 [N][K]
+    int K[6], N[6];
+    int first[6];               // first tile of each weight (the launch fills it in)
+};
+hipError_t launch_enc_prep(EncPrepArgs& a, hipStream_t s);
+hipError_t launch_enc_gather16(const int32_t* tok, int64_t rows, const int8_t* codes, const float* scales,
+                               int64_t vocab, int d, uint16_t* x16, unsigned long long* err, hipStream_t s);
+// Epilogues: f32 output matrices of D columns one after the other (Y
+// [N/D][M][D], a column scale array each); gelu and f16 output; residual +
+// layernorm, f32 and f16 output (N 128, 256 or 384); the same, the rows then
+// divided by their norm and their unmasked ones summed per column: of each
+// slab of enc_pool_slab rows, one sum per sequence it holds rows of (Y
+// [slabs][slots][N], slot 0 the sequence its first row belongs to).
+enum { ENC_EPI_F32 = 0, ENC_EPI_GELU16 = 1, ENC_EPI_LN = 2, ENC_EPI_LN_POOL = 3 };
+struct EncGemmArgs {
+    const uint16_t* A;          // f16 [M][K]
+    const uint16_t* Bt;         // f16 [N][K]
+    int64_t M;
+    int K, N, D;
+    const float* colscale[3];
+    float* Y;
+    uint16_t* Y16;
+    const float* res;           // residual [M][N], or nullptr: the q8 token rows below
+    const int32_t* tok;         // [M]
+    const int8_t* res_codes;    // [vocab][N]
+    const float* res_scales;    // [vocab]
+    int64_t vocab;
+    const int32_t* mask;        // pooled epilogue: [M]
+    int64_t T;                  // rows per sequence
+    int slots;                  // per slab: at least (slab - 1) / T + 2
+};
+int enc_pool_slab(int64_t M, int64_t d);
+hipError_t launch_enc_pool_slabs(const float* P, const int32_t* mask, int64_t b, int t, int d, int slab, int slots,
+                                 uint16_t* out, hipStream_t s);
+bool enc_ln_fused(int64_t d);
+hipError_t launch_enc_gemm16(int epi, const EncGemmArgs& a, hipStream_t s);
+// softmax(q k^T) v per sequence, q / k / v f32 [b*t][d], out f16 [b*t][d]
+bool enc_attention_supported(int64_t t, int64_t d);
+hipError_t launch_enc_attention(const float* q, const float* k, const float* v, int64_t b, int t, int d,
+                                uint16_t* out, hipStream_t s);
+
 hipError_t launch_topk_rows_partial(const float* scores, int64_t rows, int64_t cols, int64_t seg,
                                     int parts, int k, int cap, int smallest, uint64_t* partial,
                                     hipStream_t s);

@@ -1682,6 +1682,156 @@ int manta_rocm_normalize_rows(MantaRocm* rt, float* x, int64_t rows, int64_t col
     return MANTA_ROCM_OK;
 }
 
+namespace {
+
+// The encoder forward with its weight products on the f16 matrix cores (d and
+// h multiples of 128): the q8 weights widened exactly to f16 [N][K], their
+// column scales applied after the f32 accumulation, the left operands rounded
+// to f16 by the steps that produce them.  The attention products stay f32.
+// Residuals and layernorms are epilogues of the products before them (d <=
+// 384, whole rows in a tile); attention is one launch for t <= 256 and d <= 512.
+int encoder_f16(MantaRocm* rt, const int32_t* tokens, const int32_t* mask, int64_t b, int64_t t,
+                const MantaRocmEncoderWeights* w, int64_t vocab, int64_t d, int64_t h, int64_t layers, uint16_t* out,
+                char** err) {
+    const int64_t rows = b * t;
+    const bool ln = manta::enc_ln_fused(d);
+    const bool att = manta::enc_attention_supported(t, d);
+    // q, k, v [3][rows, d]; hid, y (a block's hidden rows and output) [rows,
+    // d]; x16 (the gather, then mixed, hid and y rounded) [rows, d]; ffn16
+    // [rows, h]; the weights as f16 [N][K], q, k and v one after the other.
+    // Without the fused forms also: x [rows, d], the scores [b, t, t].
+    // The column sums of the pooled rows reuse q, k and v ([slabs][slots][d]:
+    // a slab holds at least 32 rows and at most 33 sequences' shares, so even
+    // t = 1 takes less than 3 rows of d per row).
+    const size_t rd = (size_t)rows * (size_t)d;
+    const int slab = manta::enc_pool_slab(rows, d);
+    const int slots = (int)((slab - 1) / t) + 2;
+    const size_t pooled = ((size_t)rows + slab - 1) / slab * slots * d;
+    const size_t need = (2 * rd + std::max(3 * rd, pooled)) * 4 + 3 * rd * 2 + (size_t)rows * h * 2 + ((size_t)4 * d * d + (size_t)2 * d * h) * 2 +
+                        (ln ? 0 : rd * 4) + (att ? 0 : (size_t)b * t * t * 4) + 16 * 256;
+    int rc = ensure_workspace(rt, need, err);
+    if (rc) return rc;
+    Carver cv(rt->ws);
+    float* qkv = cv.take<float>(std::max(3 * rd, pooled));
+    float* hid = cv.take<float>(rd);
+    float* y = cv.take<float>(rd);
+    uint16_t* x16 = cv.take<uint16_t>(rd);
+    uint16_t* mx16 = cv.take<uint16_t>(rd);
+    uint16_t* hid16 = cv.take<uint16_t>(rd);
+    uint16_t* ffn16 = cv.take<uint16_t>((size_t)rows * h);
+    uint16_t* wq = cv.take<uint16_t>((size_t)3 * d * d);
+    uint16_t* wo = cv.take<uint16_t>((size_t)d * d);
+    uint16_t* wup = cv.take<uint16_t>((size_t)d * h);
+    uint16_t* wpr = cv.take<uint16_t>((size_t)h * d);
+    float* x = ln ? nullptr : cv.take<float>(rd);
+    float* sc = att ? nullptr : cv.take<float>((size_t)b * t * t);
+    const int D = (int)d, H = (int)h, T = (int)t;
+    hipStream_t s = rt->stream;
+
+    manta::EncPrepArgs pa{};
+    uint16_t* wt[6] = {wq, wq + d * d, wq + 2 * d * d, wo, wup, wpr};
+    for (int i = 0; i < 6; i++) {
+        pa.codes[i] = w->codes[i];
+        pa.wt[i] = wt[i];
+        pa.K[i] = i == 5 ? H : D;
+        pa.N[i] = i == 4 ? H : D;
+    }
+    LAUNCH_TRY(manta::launch_enc_prep(pa, s), "embed_transpose");
+    // (token rows not 16-byte aligned: gathered to f32 as well, the first
+    // block's residual)
+    const bool tok16 = ((uintptr_t)w->token_codes & 15) == 0;
+    if (ln && tok16)
+        LAUNCH_TRY(manta::launch_enc_gather16(tokens, rows, w->token_codes, w->token_scales, vocab, D, x16, rt->err_word, s),
+                   "encoder_gather");
+    else
+        LAUNCH_TRY(manta::launch_enc_gather_q8(tokens, rows, w->token_codes, w->token_scales, vocab, D, ln ? y : x,
+                                               rt->err_word, s, x16),
+                   "encoder_gather");
+    rt->gather_pending = true;
+    for (int64_t layer = 0; layer < layers; layer++) {
+        const bool last = layer + 1 == layers;
+        manta::EncGemmArgs ga{};
+        ga.A = x16;
+        ga.Bt = wq;
+        ga.M = rows;
+        ga.K = D;
+        ga.N = 3 * D;
+        ga.D = D;
+        for (int i = 0; i < 3; i++) ga.colscale[i] = w->col_scales[i];
+        ga.Y = qkv;
+        LAUNCH_TRY(manta::launch_enc_gemm16(manta::ENC_EPI_F32, ga, s), "encoder_gemm");
+        float *q = qkv, *k = qkv + rd, *v = qkv + 2 * rd;
+        if (att) {
+            LAUNCH_TRY(manta::launch_enc_attention(q, k, v, b, T, D, mx16, s), "encoder_attention");
+        } else {
+            // scores[b] = q[b] @ transpose(k[b]); softmax over each row of t; @ v (into q)
+            const int64_t td = (int64_t)t * d, tt = (int64_t)t * t;
+            LAUNCH_TRY(manta::launch_enc_gemm(2, q, td, k, nullptr, td, sc, tt, T, T, D, (int)b, s), "encoder_attention");
+            LAUNCH_TRY(manta::launch_enc_softmax_rows(sc, rows, T, s), "encoder_softmax");
+            LAUNCH_TRY(manta::launch_enc_gemm(0, sc, tt, v, nullptr, td, q, td, T, D, T, (int)b, s, false, mx16),
+                       "encoder_attention");
+        }
+        // attn_hidden = layernorm(mixed @ attn_o + x) (hid); the first block's
+        // x are the token rows, a later one's the last block's output
+        manta::EncGemmArgs oa{};
+        oa.A = mx16;
+        oa.Bt = wo;
+        oa.M = rows;
+        oa.K = D;
+        oa.N = oa.D = D;
+        oa.colscale[0] = w->col_scales[3];
+        oa.Y = ln ? hid : qkv;
+        oa.Y16 = hid16;
+        oa.res = layer == 0 && tok16 ? nullptr : y;
+        oa.tok = tokens;
+        oa.res_codes = w->token_codes;
+        oa.res_scales = w->token_scales;
+        oa.vocab = vocab;
+        LAUNCH_TRY(manta::launch_enc_gemm16(ln ? manta::ENC_EPI_LN : manta::ENC_EPI_F32, oa, s), "encoder_gemm");
+        if (!ln)
+            LAUNCH_TRY(manta::launch_enc_add_layernorm(qkv, layer == 0 ? x : y, hid, rows, D, s, hid16),
+                       "encoder_layernorm");
+        manta::EncGemmArgs ua{};
+        ua.A = hid16;
+        ua.Bt = wup;
+        ua.M = rows;
+        ua.K = D;
+        ua.N = H;
+        ua.colscale[0] = w->col_scales[4];
+        ua.Y16 = ffn16;
+        LAUNCH_TRY(manta::launch_enc_gemm16(manta::ENC_EPI_GELU16, ua, s), "encoder_gemm");
+        // encoded = layernorm(gelu @ projection + attn_hidden) (y and, for the
+        // next block, x16); the last block's rows are normalized too
+        manta::EncGemmArgs da{};
+        da.A = ffn16;
+        da.Bt = wpr;
+        da.M = rows;
+        da.K = H;
+        da.N = da.D = D;
+        da.colscale[0] = w->col_scales[5];
+        da.Y = ln ? (last ? qkv : y) : qkv;
+        da.Y16 = x16;
+        da.res = hid;
+        da.mask = mask;
+        da.T = t;
+        da.slots = slots;
+        LAUNCH_TRY(manta::launch_enc_gemm16(!ln ? manta::ENC_EPI_F32 : (last ? manta::ENC_EPI_LN_POOL : manta::ENC_EPI_LN),
+                                            da, s),
+                   "encoder_gemm");
+        if (!ln) LAUNCH_TRY(manta::launch_enc_add_layernorm(qkv, hid, y, rows, D, s, x16), "encoder_layernorm");
+    }
+    if (ln) {
+        LAUNCH_TRY(manta::launch_enc_pool_slabs(qkv, mask, b, T, D, slab, slots, out, s), "mean_pool");
+        return MANTA_ROCM_OK;
+    }
+    LAUNCH_TRY(manta::launch_normalize_rows(y, rows, d, s), "normalize");
+    LAUNCH_TRY(manta::launch_mean_pool_masked(y, mask, b, t, d, hid, s), "mean_pool");
+    LAUNCH_TRY(manta::launch_enc_to_f16(hid, b * d, out, s), "encoder_out");
+    return MANTA_ROCM_OK;
+}
+
+}  // namespace
+
 int manta_rocm_encoder_pooled(MantaRocm* rt, const int32_t* tokens, const int32_t* mask, int64_t b, int64_t t,
                               const MantaRocmEncoderWeights* w, int64_t vocab, int64_t d, int64_t h,
                               uint16_t* out, char** err) {
@@ -1706,23 +1856,14 @@ int manta_rocm_encoder_pooled_layers(MantaRocm* rt, const int32_t* tokens, const
     if (b > 65535 || rows > 0x7FFFFFFF || d > 0x7FFFFFFF || h > 0x7FFFFFFF || t > 0x7FFFFFFF ||
         (rows + 63) / 64 > 65535)
         return fail(err, MANTA_ROCM_UNSUPPORTED, "encoder: shape too large");
-    // The weight GEMMs run on the f16 matrix cores when d and h are multiples
-    // of 128 (embed_gemm2: the q8 weights widened exactly to f16 [N][K],
-    // their column scales applied after the f32 accumulation; the left
-    // operands rounded to f16 by the steps that produce them), else on the
-    // f32 matrix cores (enc_gemm_mfma_kernel).  The attention products stay
-    // f32.
+    // d and h multiples of 128: the weight products on the f16 matrix cores,
+    // else (here) on the f32 ones (enc_gemm_mfma_kernel)
     const bool f16w = d % 128 == 0 && h % 128 == 0 && d <= 4096 && h <= 8192;
+    if (f16w) return encoder_f16(rt, tokens, mask, b, t, w, vocab, d, h, layers, out, err);
     // x, q, k, v, mixed [rows, d]; scores [b, t, t]; ffn [rows, h]; pooled [b, d]
-    // (f16 path: x16, k16, mx16 [rows, d], ffn16 [rows, h], the six weights as f16 [N][K])
     const size_t rd = (size_t)rows * (size_t)d;
-    const size_t wsz[6] = {(size_t)d * d, (size_t)d * d, (size_t)d * d, (size_t)d * d, (size_t)d * h, (size_t)h * d};
-    const size_t ffn_f32 = f16w ? 1 : (size_t)rows * h;  // the f16 path keeps ffn in f16 only
-    size_t need = 5 * (rd * 4 + 256) + (size_t)b * t * t * 4 + 256 + ffn_f32 * 4 + 256 + (size_t)b * d * 4 + 256;
-    if (f16w) {
-        need += 3 * (rd * 2 + 256) + (size_t)rows * h * 2 + 256;
-        for (size_t z : wsz) need += z * 2 + 256;
-    }
+    const size_t need = 5 * (rd * 4 + 256) + (size_t)b * t * t * 4 + 256 + (size_t)rows * h * 4 + 256 +
+                        (size_t)b * d * 4 + 256;
     int rc = ensure_workspace(rt, need, err);
     if (rc) return rc;
     Carver cv(rt->ws);
@@ -1732,79 +1873,33 @@ int manta_rocm_encoder_pooled_layers(MantaRocm* rt, const int32_t* tokens, const
     float* v = cv.take<float>(rd);
     float* mx = cv.take<float>(rd);
     float* sc = cv.take<float>((size_t)b * t * t);
-    float* ffn = cv.take<float>(ffn_f32);
+    float* ffn = cv.take<float>((size_t)rows * h);
     float* pooled = cv.take<float>((size_t)b * d);
-    uint16_t *x16 = nullptr, *k16 = nullptr, *mx16 = nullptr, *ffn16 = nullptr, *wt[6] = {};
-    if (f16w) {
-        x16 = cv.take<uint16_t>(rd);
-        k16 = cv.take<uint16_t>(rd);
-        mx16 = cv.take<uint16_t>(rd);
-        ffn16 = cv.take<uint16_t>((size_t)rows * h);
-        for (int i = 0; i < 6; i++) wt[i] = cv.take<uint16_t>(wsz[i]);
-    }
     const int R = (int)rows, D = (int)d, H = (int)h, T = (int)t;
     const int64_t td = (int64_t)t * d, tt = (int64_t)t * t;
     hipStream_t s = rt->stream;
-    // out = in16 [R, K] x weight i (f16 [N][K], column scales) on f16 MFMA:
-    // f32 out, or f16 out with gelu applied (ffn_up)
-    auto wgemm = [&](int i, const uint16_t* in16, int K, int N, float* out, uint16_t* out16, bool gelu) {
-        manta::EmbedArgs ea{};
-        ea.A = in16;
-        ea.M = R;
-        ea.K = K;
-        ea.N = N;
-        ea.colscale = w->col_scales[i];
-        ea.Y = out;
-        ea.Y16 = out16;
-        ea.gelu = gelu ? 1 : 0;
-        return manta::launch_embed_gemm2(ea, false, true, false, wt[i], s);
-    };
-    if (f16w) {
-        const int kn[6][2] = {{D, D}, {D, D}, {D, D}, {D, D}, {D, H}, {H, D}};
-        for (int i = 0; i < 6; i++) {
-            manta::EmbedArgs ea{};
-            ea.K = kn[i][0];
-            ea.N = kn[i][1];
-            ea.B = w->codes[i];
-            LAUNCH_TRY(manta::launch_embed_transpose_b(ea, true, wt[i], s), "embed_transpose");
-        }
-    }
-    LAUNCH_TRY(manta::launch_enc_gather_q8(tokens, rows, w->token_codes, w->token_scales, vocab, D, x, rt->err_word, s,
-                                           x16),
+    LAUNCH_TRY(manta::launch_enc_gather_q8(tokens, rows, w->token_codes, w->token_scales, vocab, D, x, rt->err_word, s),
                "encoder_gather");
     rt->gather_pending = true;
     for (int64_t layer = 0; layer < layers; layer++) {
-    if (layer > 0) std::swap(x, mx);  // this block's hidden input is the last block's encoded output
-    if (f16w) {
-        LAUNCH_TRY(wgemm(0, x16, D, D, q, nullptr, false), "encoder_gemm");
-        LAUNCH_TRY(wgemm(1, x16, D, D, k, nullptr, false), "encoder_gemm");
-        LAUNCH_TRY(wgemm(2, x16, D, D, v, nullptr, false), "encoder_gemm");
-    } else {
-        LAUNCH_TRY(manta::launch_enc_gemm(1, x, 0, w->codes[0], w->col_scales[0], 0, q, 0, R, D, D, 1, s), "encoder_gemm");
-        LAUNCH_TRY(manta::launch_enc_gemm(1, x, 0, w->codes[1], w->col_scales[1], 0, k, 0, R, D, D, 1, s), "encoder_gemm");
-        LAUNCH_TRY(manta::launch_enc_gemm(1, x, 0, w->codes[2], w->col_scales[2], 0, v, 0, R, D, D, 1, s), "encoder_gemm");
-    }
-    // scores[b] = q[b] @ transpose(k[b]); softmax over each row of t
-    LAUNCH_TRY(manta::launch_enc_gemm(2, q, td, k, nullptr, td, sc, tt, T, T, D, (int)b, s), "encoder_attention");
-    LAUNCH_TRY(manta::launch_enc_softmax_rows(sc, rows, T, s), "encoder_softmax");
-    LAUNCH_TRY(manta::launch_enc_gemm(0, sc, tt, v, nullptr, td, mx, td, T, D, T, (int)b, s, false, mx16),
-               "encoder_attention");
-    // attended = mixed @ attn_o (into q); attn_hidden = layernorm(attended + x) (into k)
-    if (f16w) LAUNCH_TRY(wgemm(3, mx16, D, D, q, nullptr, false), "encoder_gemm");
-    else LAUNCH_TRY(manta::launch_enc_gemm(1, mx, 0, w->codes[3], w->col_scales[3], 0, q, 0, R, D, D, 1, s), "encoder_gemm");
-    LAUNCH_TRY(manta::launch_enc_add_layernorm(q, x, k, rows, D, s, k16), "encoder_layernorm");
-    // projected = gelu @ projection (into v); encoded = layernorm(projected + attn_hidden) (into mx, and its
-    // f16 copy into x16, the next block's input)
-    if (f16w) {
-        LAUNCH_TRY(wgemm(4, k16, D, H, nullptr, ffn16, true), "encoder_gemm");
-        LAUNCH_TRY(wgemm(5, ffn16, H, D, v, nullptr, false), "encoder_gemm");
-    } else {
+        if (layer > 0) std::swap(x, mx);  // this block's hidden input is the last block's encoded output
+        float* qkv[3] = {q, k, v};
+        for (int i = 0; i < 3; i++)
+            LAUNCH_TRY(manta::launch_enc_gemm(1, x, 0, w->codes[i], w->col_scales[i], 0, qkv[i], 0, R, D, D, 1, s),
+                       "encoder_gemm");
+        // scores[b] = q[b] @ transpose(k[b]); softmax over each row of t
+        LAUNCH_TRY(manta::launch_enc_gemm(2, q, td, k, nullptr, td, sc, tt, T, T, D, (int)b, s), "encoder_attention");
+        LAUNCH_TRY(manta::launch_enc_softmax_rows(sc, rows, T, s), "encoder_softmax");
+        LAUNCH_TRY(manta::launch_enc_gemm(0, sc, tt, v, nullptr, td, mx, td, T, D, T, (int)b, s), "encoder_attention");
+        // attended = mixed @ attn_o (into q); attn_hidden = layernorm(attended + x) (into k)
+        LAUNCH_TRY(manta::launch_enc_gemm(1, mx, 0, w->codes[3], w->col_scales[3], 0, q, 0, R, D, D, 1, s), "encoder_gemm");
+        LAUNCH_TRY(manta::launch_enc_add_layernorm(q, x, k, rows, D, s), "encoder_layernorm");
+        // projected = gelu @ projection (into v); encoded = layernorm(projected + attn_hidden) (into mx)
         LAUNCH_TRY(manta::launch_enc_gemm(1, k, 0, w->codes[4], w->col_scales[4], 0, ffn, 0, R, H, D, 1, s, true),
                    "encoder_gemm");
         LAUNCH_TRY(manta::launch_enc_gemm(1, ffn, 0, w->codes[5], w->col_scales[5], 0, v, 0, R, D, H, 1, s),
                    "encoder_gemm");
-    }
-    LAUNCH_TRY(manta::launch_enc_add_layernorm(v, k, mx, rows, D, s, x16), "encoder_layernorm");
+        LAUNCH_TRY(manta::launch_enc_add_layernorm(v, k, mx, rows, D, s), "encoder_layernorm");
     }
     LAUNCH_TRY(manta::launch_normalize_rows(mx, rows, d, s), "normalize");
     LAUNCH_TRY(manta::launch_mean_pool_masked(mx, mask, b, t, d, pooled, s), "mean_pool");

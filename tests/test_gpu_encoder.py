@@ -104,6 +104,30 @@ def test_two_layer_encoder_matches_oracle(rt, b, t, vocab, d, h):
     assert np.abs(one - got).max() > 1e-2  # the second block ran
 
 
+@pytest.mark.parametrize("layers", [1, 2])
+@pytest.mark.parametrize("b,t,vocab,d,h", [
+    # 256-row tiles with several sequences' shares in a 64-row slab, and a
+    # last tile that is not full
+    (4100, 8, 60, 128, 128),
+    # 64-row tiles: one row, sequences that cross slabs, one to five blocks of
+    # 64 positions (the last past the fused attention), d past the fused layernorm
+    (1, 1, 9, 128, 128), (3, 31, 50, 256, 384), (2, 70, 50, 256, 128), (3, 130, 80, 128, 256), (2, 200, 60, 384, 128),
+    (2, 257, 40, 128, 128), (2, 33, 40, 512, 128), (1, 20, 30, 640, 256)])
+def test_encoder_f16_tile_edges(rt, b, t, vocab, d, h, layers):
+    """The f16 weight path at the edges of its tiles, slabs and fused forms,
+    at the bar above."""
+    if b * t > 10000 and layers > 1:
+        layers = 1  # the oracle's time
+    case = _case(b * 31 + t, b, t, vocab, d, h, empty_row=b > 1)
+    got = _run_layers(rt, layers, *case).download().view(np.float16).astype(np.float32)
+    want = _want_layers(layers, *case)
+    live = np.linalg.norm(want, axis=1) > 0
+    assert np.all(got[~live] == 0.0)
+    cos = (got[live] * want[live]).sum(1) / (np.linalg.norm(got[live], axis=1) * np.linalg.norm(want[live], axis=1))
+    assert cos.min() >= 0.9999, cos.min()
+    assert np.abs(got - want).max() < 2e-3
+
+
 def test_encoder_output_feeds_score_topk(rt):
     """The encoder's device output is the query matrix of the fused score +
     top-k with no host round trip; the result equals the reference scoring
