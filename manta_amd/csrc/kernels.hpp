@@ -20,6 +20,8 @@ struct QConst;
 constexpr int kMaxQueryDim = 1024;  // longest query / row the device path takes
 constexpr int kMaxCapKeys = 4096;   // largest LDS key reservoir (32 KB)
 constexpr int kWaveListMaxK = 64;   // largest k kept in per-wave register lists
+constexpr int kBestMaxK = 192;      // largest k selected by a floor and ranks (best_common.hpp)
+constexpr int kBestMaxParts = 512;  // parts such a merge takes
 
 // Arguments of the streaming scan kernels (one query per blockIdx.y).
 struct ScanArgs {
@@ -45,6 +47,8 @@ struct ScanArgs {
     int mid_compact;          // 0: cap >= k + rounds*256, no compaction between rounds
     int smallest;
     int wave_lists;           // 1: k <= 64 top lists held in registers (coalesced q8 kernel only)
+    int buffered;             // 1: k <= kBestMaxK, every score kept in LDS ([rounds][256] words at the front of
+                              // the dynamic LDS) and selected at the end (lds_keys = rounds * 128)
 };
 
 // Query codes for the batched paths (one workgroup per query).  With tau

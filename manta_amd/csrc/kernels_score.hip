@@ -25,6 +25,7 @@
 // The E16 scores rank rows for the reference-semantics top-k, which
 // rescores the best of them with the reference's arithmetic
 // (kernels_ref.hip).
+#include "best_common.hpp"
 #include "device_common.hpp"
 #include "kernels.hpp"
 #include "q4_common.hpp"
@@ -239,16 +240,54 @@ struct ScanLds {
     int last;
 };
 
-// Store the score, or offer it to the reservoir.
-__device__ __forceinline__ void emit_round(float score, bool valid, int64_t row, int64_t n, int qi,
-                                           float* __restrict__ out_scores, uint64_t* keys,
-                                           TopKShared* st, uint64_t tau, int smallest) {
-    if (out_scores) {
-        if (valid) out_scores[(int64_t)qi * n + row] = score;
+// One round's score of this thread's row (round r of the workgroup): stored,
+// buffered for finish_buffered, or offered to the reservoir.
+__device__ __forceinline__ void emit_round(const ScanArgs& a, float score, bool valid, int64_t row, int r, int qi,
+                                           uint64_t* keys, TopKShared* st) {
+    if (a.out_scores) {
+        if (valid) a.out_scores[(int64_t)qi * a.n + row] = score;
         return;
     }
-    uint64_t key = valid ? make_key(score, (uint32_t)row, smallest) : 0ull;
-    topk_offer(key, tau, keys, st);
+    if (a.buffered) {
+        const uint32_t o = float_order(score);
+        ((uint32_t*)keys)[r * 256 + threadIdx.x] = valid ? (a.smallest ? ~o : o) : 0u;
+        return;
+    }
+    const uint64_t key = valid ? make_key(score, (uint32_t)row, a.smallest) : 0ull;
+    topk_offer(key, st->tau, keys, st);
+    if (a.mid_compact) {
+        __syncthreads();
+        topk_maybe_compact(keys, st, a.k, a.cap);
+    }
+}
+
+// End of a buffered top-k scan workgroup (64 < k <= kBestMaxK): its scores
+// are in LDS, a thread's own rows in its own words, so the rounds ran without
+// a barrier or an atomic; the k best of them, and of the query's parts, by a
+// floor and ranks.  Against the reservoir (compactions between rounds, the
+// last workgroup streaming every part key through it): one q4 query, 1,048,576
+// rows, k = 108, 159 -> 57 us.
+__device__ __forceinline__ void finish_buffered(const ScanArgs& a, const uint64_t* buf, int qi) {
+    __shared__ BestShared B;
+    const uint32_t* slots = (const uint32_t*)buf;  // (rows past n: 0)
+    const int tid = threadIdx.x;
+    const int64_t row0 = (int64_t)blockIdx.x * a.rounds * 256;
+    const int left = a.n - row0 < (int64_t)a.rounds * 256 ? (int)(a.n - row0) : a.rounds * 256;
+    int kept = block_best<0>([&](int j) { return slots[j * 256 + tid]; },
+                             [&](int j) { return j * 256 + tid < left ? (int)(row0 + j * 256 + tid) : -1; }, a.rounds,
+                             a.k, B);
+    if (kept < 0)
+        kept = best_streamed([&](int64_t i) { return ((uint64_t)slots[i] << 32) | (uint64_t)(~(uint32_t)(row0 + i)); },
+                             left, 1ull, a.k, B);
+    if (gridDim.x > 1) {
+        kept = merge_best_parts(a.partial, a.tickets, qi, kept, a.k, B);
+        if (kept < 0) return;
+    }
+    for (int i = tid; i < a.k; i += 256) {
+        const uint64_t e = i < kept ? B.keys[i] : 0ull;
+        a.out_ids[(int64_t)qi * a.k + i] = e ? (int32_t)key_index(e) : -1;
+        if (a.out_topk_scores) a.out_topk_scores[(int64_t)qi * a.k + i] = e ? key_score(e, a.smallest) : 0.0f;
+    }
 }
 
 // End of a top-k scan workgroup on the wave-list path (k <= 64): the waves'
@@ -501,8 +540,12 @@ __device__ __forceinline__ QConst encode_query_lanes(const uint16_t* qrow, int d
 // accumulator of its own row.  Loads go through a buffer resource clipped to
 // the workgroup's rows (no branch per load; rows past n read zero and are
 // masked by `valid`).
-template <int OP, int L, int C, bool LISTS>
+enum { SCAN_RESERVOIR = 0, SCAN_LISTS = 1, SCAN_BUFFERED = 2 };
+
+template <int OP, int L, int C, int MODE>
 __global__ __launch_bounds__(256) void q8_scan_kernel(ScanArgs a) {
+    constexpr bool LISTS = MODE == SCAN_LISTS;
+    constexpr bool AHEAD = MODE != SCAN_RESERVOIR;  // the next step's loads go out early
     extern __shared__ uint64_t topk_keys[];
     __shared__ ScanTopkLds S;
     __shared__ uint64_t ff_keys[LISTS ? 256 : 1];  // the lists' first fill, 64 keys a wave
@@ -525,7 +568,7 @@ __global__ __launch_bounds__(256) void q8_scan_kernel(ScanArgs a) {
     const __amdgpu_buffer_rsrc_t rs = byte_buffer(codes + wg_row0 * PITCH, (uint32_t)wg_rows * PITCH);
     const int lane_off = g * L * PITCH + p * 16;
     // One load step: rows j0 .. j0+JS-1 of every lane group of the wave's
-    // block in round r.  On the wave-list path the next step's loads are
+    // block in round r.  On the list and buffered paths the next step's loads are
     // issued as soon as the current step's values are consumed, so they
     // overlap the epilogue and the top-k offer, and the first step's overlap
     // the query encoding.
@@ -538,13 +581,13 @@ __global__ __launch_bounds__(256) void q8_scan_kernel(ScanArgs a) {
             for (int c = 0; c < C; c++)
                 v[j][c] = __builtin_amdgcn_raw_buffer_load_b128(rs, vb + (j0 + j) * PITCH + c * 16 * L, 0, 2);
     };
-    if (LISTS) load_step(0, 0);
+    if (AHEAD) load_step(0, 0);
 
     v4i qa[C], qb[C];
     const QConst kq = encode_query_lanes<OP, L, C>(a.queries + (int64_t)qi * a.d, a.d, p, qa, qb);
     // LISTS: top-k through per-wave register lists (k <= 64, never score mode)
     uint64_t list = 0, thr = 0;
-    if (!LISTS && !a.out_scores) topk_init(topk_keys, &S.st);
+    if (MODE == SCAN_RESERVOIR && !a.out_scores) topk_init(topk_keys, &S.st);
 
     for (int r = 0; r < a.rounds; r++) {
         const int64_t row = wg_row0 + r * 256 + wave * 64 + lane;
@@ -559,7 +602,7 @@ __global__ __launch_bounds__(256) void q8_scan_kernel(ScanArgs a) {
         for (int j0 = 0; j0 < L; j0 += JS) {
             // the reservoir path loads each step when it starts (its offer
             // and compaction would otherwise run with a step of loads held)
-            if (!LISTS) load_step(r, j0);
+            if (!AHEAD) load_step(r, j0);
 #pragma unroll
             for (int j = 0; j < JS; j++) {
                 int s_hi = 0, s_lo = 0;
@@ -580,7 +623,7 @@ __global__ __launch_bounds__(256) void q8_scan_kernel(ScanArgs a) {
             // registers held)
             asm volatile("" : "+v"(my_hi), "+v"(my_lo));
             asm volatile("" ::: "memory");
-            if (!LISTS) continue;
+            if (!AHEAD) continue;
             // unconditional, so the wait counts stay static: after the last
             // round these loads fall past the buffer and return zeros
             // without touching memory
@@ -600,103 +643,223 @@ __global__ __launch_bounds__(256) void q8_scan_kernel(ScanArgs a) {
             else wave_list_offer(key, list, thr, a.k);
             continue;
         }
-        const uint64_t tau = a.out_scores ? 0ull : S.st.tau;
-        emit_round(score, valid, row, a.n, qi, a.out_scores, topk_keys, &S.st, tau, a.smallest);
-        if (!a.out_scores && a.mid_compact) {
-            __syncthreads();
-            topk_maybe_compact(topk_keys, &S.st, a.k, a.cap);
-        }
+        emit_round(a, score, valid, row, r, qi, topk_keys, &S.st);
     }
     if (LISTS)
         finish_wave_lists(a, list, thr, topk_keys, S, qi);
+    else if (MODE == SCAN_BUFFERED)
+        finish_buffered(a, topk_keys, qi);
     else if (!a.out_scores)
         finish_topk(a, topk_keys, S, qi);
 }
 
-// --------------------------------------------- q8, any pitch (lane = row)
+// ------------------------------------------ q8, any pitch (lane = 16 bytes)
 
+// LDS words (int2) a wave of the kernel below trades sums through: 8 loads of
+// 64 / nc rows, nc | 1 words each (rows on distinct banks).
+__host__ __device__ constexpr int q8_generic_words(int nc) { return 8 * (64 / nc) * (nc | 1); }
+
+// Lane p of a group of pitch/16 lanes takes bytes [16p, +16) of a row, so a
+// load instruction reads 64 / (pitch/16) whole rows side by side; the lanes'
+// integer sums meet through LDS, one lane adding a row's, a batch of 8 loads at
+// a time, and lane i of the wave keeps row i of its 64.  Loads are 8
+// instructions ahead, across rounds too.  (A row per lane read 16 bytes out of
+// every row per load: two queries over 300,000 rows of 1,000, k = 180, 303 us
+// a call against 173.)
 template <int OP>
 __global__ __launch_bounds__(256) void q8_scan_generic_kernel(ScanArgs a) {
     extern __shared__ uint64_t topk_keys[];
     __shared__ ScanLds S;
+    __shared__ int2 sums[4][64];  // a wave's row sums of the round
+    constexpr int B = 8;
     const int qi = blockIdx.y;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nc = a.pitch / 16;
+    const int rpl = 64 / nc, steps = (64 + rpl - 1) / rpl;  // rows per load, loads per 64 rows
+    const int g = lane / nc, p = lane - g * nc;
+    const bool act = g < rpl;
     const int64_t set_row0 = (int64_t)qi * a.set_stride;
-    const int8_t* __restrict__ codes = a.codes + set_row0 * a.pitch;
     const float* __restrict__ scales = (const float*)a.scales + set_row0;
+    const int64_t wg_row0 = (int64_t)blockIdx.x * a.rounds * 256;
+    const int64_t left = a.n - wg_row0;  // > 0: the grid covers n exactly
+    const int wg_rows = left < (int64_t)a.rounds * 256 ? (int)left : a.rounds * 256;
+    const __amdgpu_buffer_rsrc_t rs =
+        byte_buffer(a.codes + (set_row0 + wg_row0) * a.pitch, (uint32_t)wg_rows * a.pitch);
+    // past the buffer, whatever row is added: such loads touch no memory
+    constexpr int kFar = 0x40000000;
+    const int voff = act ? (wave * 64 + g) * a.pitch + p * 16 : kFar;
+    v4i w[B], wn[B];
+    auto load = [&](v4i (&dw)[B], int r, int s0) {
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            const bool in = s0 + j < steps;  // the same for the whole wave
+            dw[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, in ? (r * 256 + (s0 + j) * rpl) * a.pitch : kFar, 2);
+        }
+    };
+    load(w, 0, 0);
     encode_query_block(a.queries + (int64_t)qi * a.d, a.d, a.pitch, OP == OP_DOT ? ENC_E8 : ENC_E16, S.q);
     const QConst kq = S.q.qc;
-    const int8_t* qa = OP == OP_DOT ? S.q.c8 : S.q.hi;
-    const int8_t* qb = S.q.lo;
-    const int chunks = a.pitch / 16;
-    if (!a.out_scores) topk_init(topk_keys, &S.st);
-    const int64_t wg_row0 = (int64_t)blockIdx.x * a.rounds * 256;
+    const v4i qa = *(const v4i*)((OP == OP_DOT ? S.q.c8 : S.q.hi) + 16 * p);
+    const v4i qb = OP == OP_DOT ? qa : *(const v4i*)(S.q.lo + 16 * p);
+    const int pp = nc | 1;
+    const int H = rpl == 1 ? 8 : (rpl == 2 ? 4 : (rpl <= 4 ? 2 : 1));  // H * 8 * rpl <= 64
+    int2* part = (int2*)(topk_keys + a.lds_keys) + wave * q8_generic_words(nc);
+    if (!a.out_scores && !a.buffered) topk_init(topk_keys, &S.st);
     for (int r = 0; r < a.rounds; r++) {
-        const int64_t row = wg_row0 + (int64_t)r * 256 + threadIdx.x;
+        const int64_t row = wg_row0 + (int64_t)r * 256 + wave * 64 + lane;
         const bool valid = row < a.n;
-        int s_hi = 0, s_lo = 0;
-        if (valid) {
-            const v4i* rp = (const v4i*)(codes + row * a.pitch);
-            for (int c = 0; c < chunks; c++) {
-                v4i v = rp[c];
-                s_hi = dot16(v, *(const v4i*)(qa + c * 16), s_hi);
-                if (OP != OP_DOT) s_lo = dot16(v, *(const v4i*)(qb + c * 16), s_lo);
+        const int64_t crow = valid ? row : a.n - 1;
+        const float sc = scales[crow];
+        const float dn = OP == OP_COSINE ? a.dnorm[set_row0 + crow] : 0.0f;
+        const float d2 = OP == OP_L2 ? a.dd[set_row0 + crow] : 0.0f;
+        for (int s0 = 0; s0 < steps; s0 += B) {
+            const bool more = s0 + B < steps;
+            load(wn, more ? r : r + 1, more ? s0 + B : 0);
+#pragma unroll
+            for (int j = 0; j < B; j++) {
+                const int hi = dot16(w[j], qa, 0);
+                const int lo = OP == OP_DOT ? 0 : dot16(w[j], qb, 0);
+                if (act) part[(j * rpl + g) * pp + p] = int2{hi, lo};
             }
+#pragma unroll
+            for (int j = 0; j < B; j++) w[j] = wn[j];
+            // the wave's lanes trade sums: its LDS operations run in order,
+            // the empty asm statements keep the compiler to that order
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("" ::: "memory");
+            if (H == 1) {
+                for (int br = lane; br < B * rpl; br += 64) {
+                    int2 t{0, 0};
+#pragma unroll 4
+                    for (int c = 0; c < nc; c++) {
+                        const int2 e = part[br * pp + c];
+                        t.x += e.x, t.y += e.y;
+                    }
+                    if (s0 * rpl + br < 64) sums[wave][s0 * rpl + br] = t;
+                }
+            } else {
+                // few wide rows: H lanes share a row's words
+                const int br = lane / H;
+                int2 t{0, 0};
+                if (br < B * rpl) {
+#pragma unroll 4
+                    for (int c = lane & (H - 1); c < nc; c += H) {
+                        const int2 e = part[br * pp + c];
+                        t.x += e.x, t.y += e.y;
+                    }
+                }
+                for (int off = 1; off < H; off <<= 1) {
+                    t.x += __shfl_xor(t.x, off);
+                    t.y += __shfl_xor(t.y, off);
+                }
+                if ((lane & (H - 1)) == 0 && br < B * rpl && s0 * rpl + br < 64) sums[wave][s0 * rpl + br] = t;
+            }
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("" ::: "memory");
         }
-        float score = 0.0f;
-        if (valid) {
-            float dn = 0.0f, d2 = 0.0f;
-            if (OP == OP_COSINE) dn = a.dnorm[set_row0 + row];
-            if (OP == OP_L2) d2 = a.dd[set_row0 + row];
-            score = q8_epilogue<OP>(s_hi, s_lo, scales[row], kq, dn, d2);
-        }
-        const uint64_t tau = a.out_scores ? 0ull : S.st.tau;
-        emit_round(score, valid, row, a.n, qi, a.out_scores, topk_keys, &S.st, tau, a.smallest);
-        if (!a.out_scores && a.mid_compact) {
-            __syncthreads();
-            topk_maybe_compact(topk_keys, &S.st, a.k, a.cap);
-        }
+        const int2 acc = sums[wave][lane];
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("" ::: "memory");
+        const float score = valid ? q8_epilogue<OP>(acc.x, acc.y, sc, kq, dn, d2) : 0.0f;
+        emit_round(a, score, valid, row, r, qi, topk_keys, &S.st);
     }
-    if (!a.out_scores) finish_topk(a, topk_keys, S, qi);
+    if (a.buffered) finish_buffered(a, topk_keys, qi);
+    else if (!a.out_scores) finish_topk(a, topk_keys, S, qi);
 }
 
-// ------------------------------------------------------- q4 (lane = row)
+// ------------------------------------------------------- q4, lane = block
 
-// Each thread scores one row per round (q4_row_dotf); the query digit
-// planes are permuted to the nibble order (q4_perm_pos).
+// Lane p of a group of nb lanes takes block p of a row, so a load instruction
+// reads 64 / nb whole rows side by side (16 bytes a lane, the block's f16 scale
+// beside it) and the lane's 32 query codes stay in registers.  The contract's
+// fma chain runs over a row's blocks in order, so the block sums go through
+// LDS as (scale, sum) pairs and lane i of the wave folds row i of its 64 (pair
+// pitch nb | 1: 64 rows on distinct banks).  Loads are 8 instructions ahead,
+// across rounds too.  The read of the rows bounds it: one query against
+// 1,048,576 x 384 rows took 167 us with a row per lane (16 bytes out of every
+// 192 per load), 57 this way with the selection (226 MB: 46 us at the copy
+// rate).
 template <int OP>
 __global__ __launch_bounds__(256) void q4_scan_kernel(ScanArgs a) {
     extern __shared__ uint64_t topk_keys[];
     __shared__ ScanLds S;
+    constexpr int B = 8;
     const int qi = blockIdx.y;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nb = a.nb;
+    const int rpl = 64 / nb, steps = (64 + rpl - 1) / rpl;  // rows per load, loads per 64 rows
+    const int g = lane / nb, p = lane - g * nb;
+    const bool act = g < rpl;
     const int64_t set_row0 = (int64_t)qi * a.set_stride;
-    const uint8_t* __restrict__ packed = (const uint8_t*)a.codes + set_row0 * a.pitch;
-    const uint16_t* __restrict__ scales = (const uint16_t*)a.scales + set_row0 * a.nb;
+    const int64_t wg_row0 = (int64_t)blockIdx.x * a.rounds * 256;
+    const int64_t left = a.n - wg_row0;  // > 0: the grid covers n exactly
+    const int wg_rows = left < (int64_t)a.rounds * 256 ? (int)left : a.rounds * 256;
+    const __amdgpu_buffer_rsrc_t rs =
+        byte_buffer((const uint8_t*)a.codes + (set_row0 + wg_row0) * a.pitch, (uint32_t)wg_rows * a.pitch);
+    const __amdgpu_buffer_rsrc_t ss =
+        byte_buffer((const uint16_t*)a.scales + (set_row0 + wg_row0) * nb, (uint32_t)wg_rows * nb * 2);
+    // past every buffer, whatever row is added: such loads touch no memory
+    constexpr int kFar = 0x40000000;
+    const int voff = act ? (wave * 64 + g) * a.pitch + p * 16 : kFar;
+    const int soff = act ? ((wave * 64 + g) * nb + p) * 2 : kFar;
+    v4i w[B], wn[B];
+    uint16_t sc[B], scn[B];
+    auto load = [&](v4i (&dw)[B], uint16_t (&ds)[B], int r, int s0) {
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            const int row = r * 256 + (s0 + j) * rpl;
+            const bool in = s0 + j < steps;  // the same for the whole wave
+            dw[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, in ? row * a.pitch : kFar, 2);
+            ds[j] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(ss, soff, in ? row * nb * 2 : kFar, 2);
+        }
+    };
+    load(w, sc, 0, 0);
     encode_query_block(a.queries + (int64_t)qi * a.d, a.d, a.d, ENC_E16_Q4, S.q);
     const QConst kq = S.q.qc;
-    const int* qh = (const int*)S.q.hi;
-    const int* ql = (const int*)S.q.lo;
-    if (!a.out_scores) topk_init(topk_keys, &S.st);
-    const int64_t wg_row0 = (int64_t)blockIdx.x * a.rounds * 256;
-    for (int r = 0; r < a.rounds; r++) {
-        const int64_t row = wg_row0 + (int64_t)r * 256 + threadIdx.x;
-        const bool valid = row < a.n;
-        float dotf = 0.0f;
-        if (valid) dotf = q4_row_dotf(packed + row * a.pitch, scales + row * a.nb, a.nb, qh, ql);
-        float score = 0.0f;
-        if (valid) {
-            float dn = 0.0f, d2 = 0.0f;
-            if (OP == OP_COSINE) dn = a.dnorm[set_row0 + row];
-            if (OP == OP_L2) d2 = a.dd[set_row0 + row];
-            score = q4_finish<OP>(dotf, kq, dn, d2);
-        }
-        const uint64_t tau = a.out_scores ? 0ull : S.st.tau;
-        emit_round(score, valid, row, a.n, qi, a.out_scores, topk_keys, &S.st, tau, a.smallest);
-        if (!a.out_scores && a.mid_compact) {
-            __syncthreads();
-            topk_maybe_compact(topk_keys, &S.st, a.k, a.cap);
-        }
+    int qh[8], ql[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        qh[j] = ((const int*)S.q.hi)[8 * p + j];
+        ql[j] = ((const int*)S.q.lo)[8 * p + j];
     }
-    if (!a.out_scores) finish_topk(a, topk_keys, S, qi);
+    const int pp = nb | 1;
+    float2* pairs = (float2*)(topk_keys + a.lds_keys) + wave * 64 * pp;
+    if (!a.out_scores && !a.buffered) topk_init(topk_keys, &S.st);
+    for (int r = 0; r < a.rounds; r++) {
+        const int64_t row = wg_row0 + (int64_t)r * 256 + wave * 64 + lane;
+        const bool valid = row < a.n;
+        const int64_t crow = set_row0 + (valid ? row : a.n - 1);
+        const float dn = OP == OP_COSINE ? a.dnorm[crow] : 0.0f;
+        const float d2 = OP == OP_L2 ? a.dd[crow] : 0.0f;
+        for (int s0 = 0; s0 < steps; s0 += B) {
+            const bool more = s0 + B < steps;
+            load(wn, scn, more ? r : r + 1, more ? s0 + B : 0);
+#pragma unroll
+            for (int j = 0; j < B; j++) {
+                const int lr = (s0 + j) * rpl + g;  // row of the wave's 64
+                const float acc = (float)q4_block_acc(w[j], qh, ql);
+                if (act && lr < 64) pairs[lr * pp + p] = float2{h2f(sc[j]), acc};
+            }
+#pragma unroll
+            for (int j = 0; j < B; j++) w[j] = wn[j], sc[j] = scn[j];
+        }
+        // the wave's lanes trade pairs: its LDS operations run in order, the
+        // empty asm statements keep the compiler to that order
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("" ::: "memory");
+        float dotf = 0.0f;
+#pragma unroll 4
+        for (int b = 0; b < nb; b++) {
+            const float2 e = pairs[lane * pp + b];
+            dotf = __fmaf_rn(e.x, e.y, dotf);
+        }
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("" ::: "memory");
+        const float score = valid ? q4_finish<OP>(dotf, kq, dn, d2) : 0.0f;
+        emit_round(a, score, valid, row, r, qi, topk_keys, &S.st);
+    }
+    if (a.buffered) finish_buffered(a, topk_keys, qi);
+    else if (!a.out_scores) finish_topk(a, topk_keys, S, qi);
 }
 
 // ------------------------------------------------ exact accumulator rescore
@@ -754,11 +917,13 @@ static hipError_t launch_q8_op(const ScanArgs& a, dim3 grid, size_t lds, hipStre
     if (a.wave_lists && !a.out_scores && lds < 256 * sizeof(uint64_t)) return hipErrorInvalidValue;
 #define MANTA_Q8(LL, CC)                                                                           \
     if (chunks == (LL) * (CC)) {                                                                   \
-        if (a.wave_lists && !a.out_scores)                                                         \
-            hipLaunchKernelGGL((q8_scan_kernel<OP, LL, CC, true>), grid, dim3(256), lds, s, a);  \
-        else                                                                                       \
-            hipLaunchKernelGGL((q8_scan_kernel<OP, LL, CC, false>), grid, dim3(256), lds, s, a); \
-        return hipGetLastError();                                                                  \
+        if (a.wave_lists && !a.out_scores)                                                                    \
+            hipLaunchKernelGGL((q8_scan_kernel<OP, LL, CC, SCAN_LISTS>), grid, dim3(256), lds, s, a);        \
+        else if (a.buffered && !a.out_scores)                                                                 \
+            hipLaunchKernelGGL((q8_scan_kernel<OP, LL, CC, SCAN_BUFFERED>), grid, dim3(256), lds, s, a);     \
+        else                                                                                                  \
+            hipLaunchKernelGGL((q8_scan_kernel<OP, LL, CC, SCAN_RESERVOIR>), grid, dim3(256), lds, s, a);    \
+        return hipGetLastError();                                                                             \
     }
     MANTA_Q8(4, 1)    // d <= 64
     MANTA_Q8(8, 1)    // 128
@@ -769,7 +934,9 @@ static hipError_t launch_q8_op(const ScanArgs& a, dim3 grid, size_t lds, hipStre
     MANTA_Q8(16, 3)   // 768
     MANTA_Q8(16, 4)   // 1024
 #undef MANTA_Q8
-    hipLaunchKernelGGL((q8_scan_generic_kernel<OP>), grid, dim3(256), lds, s, a);
+    if (chunks < 1 || chunks > 64 || a.pitch != 16 * chunks || lds < (size_t)a.lds_keys * 8) return hipErrorInvalidValue;
+    const size_t all = (size_t)a.lds_keys * 8 + (size_t)4 * q8_generic_words(chunks) * sizeof(int2);
+    hipLaunchKernelGGL((q8_scan_generic_kernel<OP>), grid, dim3(256), all, s, a);
     return hipGetLastError();
 }
 
@@ -783,10 +950,12 @@ hipError_t launch_q8_scan(int op, const ScanArgs& a, dim3 grid, size_t lds, hipS
 }
 
 hipError_t launch_q4_scan(int op, const ScanArgs& a, dim3 grid, size_t lds, hipStream_t s) {
+    if (a.nb < 1 || a.nb > 32 || a.pitch != 16 * a.nb || lds < (size_t)a.lds_keys * 8) return hipErrorInvalidValue;
+    const size_t all = (size_t)a.lds_keys * 8 + (size_t)4 * 64 * (a.nb | 1) * sizeof(float2);  // + (scale, sum) pairs
     switch (op) {
-        case OP_DOT: hipLaunchKernelGGL((q4_scan_kernel<OP_DOT>), grid, dim3(256), lds, s, a); break;
-        case OP_COSINE: hipLaunchKernelGGL((q4_scan_kernel<OP_COSINE>), grid, dim3(256), lds, s, a); break;
-        default: hipLaunchKernelGGL((q4_scan_kernel<OP_L2>), grid, dim3(256), lds, s, a); break;
+        case OP_DOT: hipLaunchKernelGGL((q4_scan_kernel<OP_DOT>), grid, dim3(256), all, s, a); break;
+        case OP_COSINE: hipLaunchKernelGGL((q4_scan_kernel<OP_COSINE>), grid, dim3(256), all, s, a); break;
+        default: hipLaunchKernelGGL((q4_scan_kernel<OP_L2>), grid, dim3(256), all, s, a); break;
     }
     return hipGetLastError();
 }

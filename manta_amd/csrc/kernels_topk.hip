@@ -9,120 +9,18 @@
 // Results are sorted by (value desc, index asc) -- or (value asc, index asc)
 // for smallest-k.  Keys make the order total, so the result does not
 // depend on how rows were split across workgroups.
+#include "best_common.hpp"
 #include "device_common.hpp"
 #include "kernels.hpp"
-#include "mq_common.hpp"
 
 namespace manta {
-
-namespace {
-
-constexpr int kBestKeys = 1024;  // LDS keys of block_best
-constexpr int kBestMaxK = 192;   // largest k it takes
-constexpr int kMergeKeys = 4096;  // keys a merging workgroup holds (16 a thread)
-
-struct BestShared {
-    alignas(16) uint64_t keys[kBestKeys];
-    TopKShared st;
-    uint32_t floor;
-    int cnt;
-    int last;
-};
-
-// Keys above `mine` among keys[0..n) (n a multiple of 2; every lane reads the
-// same address: LDS broadcasts, no dependent steps).
-__device__ __forceinline__ int rank_in(const uint64_t* keys, int n, uint64_t mine) {
-    int rank = 0;
-#pragma unroll 16
-    for (int i = 0; i < n; i += 2) {
-        const ulonglong2 u = *(const ulonglong2*)(keys + i);
-        rank += (u.x > mine ? 1 : 0) + (u.y > mine ? 1 : 0);
-    }
-    return rank;
-}
-
-// The best min(k, held) of the workgroup's keys, sorted, to B.keys (k <=
-// kBestMaxK; 256 threads, V keys each: held(j) the thread's j-th, 0 = none,
-// from registers; again(j) the same from memory).  The k-th largest of the
-// 256 threads' own best scores is a floor of the k-th (k distinct keys reach
-// it), and few others do: 126 of 8,192 evenly spread keys for k = 100.
-// Those take their place by rank, with no round of histograms and no sort.
-// Keys so arranged that more than kBestKeys reach the floor go through the
-// reservoir.  Returns how many keys are left.
-template <int V, class H, class A>
-__device__ __forceinline__ int block_best(H held, A again, int k, BestShared& B) {
-    const int tid = threadIdx.x;
-    // the floor needs the keys' score halves only
-    uint32_t best = 0;
-#pragma unroll
-    for (int j = 0; j < V; j++) {
-        const uint32_t o = (uint32_t)(held(j) >> 32);
-        best = o > best ? o : best;
-    }
-    uint32_t* tops = (uint32_t*)B.keys;
-    tops[tid] = best;
-    if (tid == 0) {
-        B.floor = 0u;
-        B.cnt = 0;
-    }
-    __syncthreads();
-    int above = 0, reach = 0;  // threads whose best is above, at least, this thread's
-#pragma unroll 16
-    for (int i = 0; i < 256; i += 4) {
-        const uint4 u = *(const uint4*)(tops + i);
-        above += (u.x > best ? 1 : 0) + (u.y > best ? 1 : 0) + (u.z > best ? 1 : 0) + (u.w > best ? 1 : 0);
-        reach += (u.x >= best ? 1 : 0) + (u.y >= best ? 1 : 0) + (u.z >= best ? 1 : 0) + (u.w >= best ? 1 : 0);
-    }
-    if (above < k && reach >= k) B.floor = best;  // every writer's value is the same
-    __syncthreads();
-    const uint64_t tau = ((uint64_t)B.floor << 32) | 1ull;  // (a key's low half is never 0)
-    int mine = 0;
-#pragma unroll
-    for (int j = 0; j < V; j++) mine += held(j) >= tau ? 1 : 0;
-    int pos = wave_append(mine, &B.cnt);
-    __syncthreads();
-    const int total = B.cnt;
-    if (total <= kBestKeys) {
-#pragma unroll
-        for (int j = 0; j < V; j++) {
-            const uint64_t key = held(j);
-            if (key >= tau) B.keys[pos++] = key;
-        }
-        if (total <= 256) {
-            if (tid == 0 && (total & 1)) B.keys[total] = 0ull;  // rank_in reads pairs
-            __syncthreads();
-            const uint64_t key = tid < total ? B.keys[tid] : 0ull;
-            const int rank = rank_in(B.keys, (total + 1) & ~1, key);
-            __syncthreads();
-            if (tid < total && rank < k) B.keys[rank] = key;
-            __syncthreads();
-            return total < k ? total : k;
-        }
-        if (tid == 0) B.st.cnt = total;
-        __syncthreads();
-    } else {
-        topk_init(B.keys, &B.st);
-        for (int j = 0; j < V; j++) {
-            const uint64_t t = B.st.tau > tau - 1 ? B.st.tau : tau - 1;
-            topk_offer(again(j), t, B.keys, &B.st);
-            __syncthreads();
-            topk_maybe_compact(B.keys, &B.st, k, kBestKeys);
-        }
-    }
-    topk_compact(B.keys, &B.st, k);
-    const int kept = B.st.cnt;
-    topk_sort(B.keys, kept);
-    return kept;
-}
-
-}  // namespace
 
 // One workgroup per segment of 256*V scores, one launch for the whole top-k:
 // the last workgroup of a row (ticket) merges the parts.  Publication as in
 // finish_topk: agent-scope part stores, retired before the ticket.  What
 // bounds it is the read of the scores; the streaming reservoir (a barrier
 // pair per 256 scores) and its merge launch took 62 + 27 us for 64 rows of
-// 200,000 and k = 100, this kernel 50 us.
+// 200,000 and k = 100, this kernel 26 us.
 template <int V, bool VEC>
 __global__ __launch_bounds__(256) void topk_rows_kernel(const float* __restrict__ scores, int64_t cols, int k,
                                                         int smallest, uint64_t* __restrict__ partial,
@@ -155,42 +53,18 @@ __global__ __launch_bounds__(256) void topk_rows_kernel(const float* __restrict_
         o[j] = float_order(__uint_as_float(o[j]));
         if (smallest) o[j] = ~o[j];
     }
-    auto held = [&](int j) {
-        const int c = at(j);
-        return c < left ? ((uint64_t)o[j] << 32) | (uint64_t)(~(uint32_t)(c0 + c)) : 0ull;
-    };
-    auto again = [&](int j) {
-        const int c = at(j);
-        return c < left ? make_key(src[c0 + c], (uint32_t)(c0 + c), smallest) : 0ull;
-    };
-    int kept = block_best<V>(held, again, k, B);
-    if (P > 1) {
-        uint64_t* part = partial + row * P * k;
-        uint64_t* dst = part + (int64_t)blockIdx.x * k;
-        for (int i = tid; i < k; i += 256)
-            __hip_atomic_store(dst + i, i < kept ? B.keys[i] : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (tid == 0)
-            B.last = __hip_atomic_fetch_add(&tickets[row], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                     (uint32_t)(P - 1);
-        __syncthreads();
-        if (!B.last) return;
-        // the parts' keys rank by rank (the parts are sorted), so the best of
-        // them are spread over all threads
-        const int M = P * k;  // <= kMergeKeys
-        auto load = [&](int j) {
-            const int i = tid + 256 * j;
-            if (i >= M) return (uint64_t)0;
-            const int r = i / P, p = i - r * P;
-            return (uint64_t)__hip_atomic_load(part + (int64_t)p * k + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        };
-        constexpr int MV = kMergeKeys / 256;
-        uint64_t kk[MV];
+    if (left < 256 * V) {
 #pragma unroll
-        for (int j = 0; j < MV; j++) kk[j] = load(j);
-        kept = block_best<MV>([&](int j) { return kk[j]; }, load, k, B);
-        if (tid == 0) __hip_atomic_store(&tickets[row], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int j = 0; j < V; j++) o[j] = at(j) < left ? o[j] : 0u;
+    }
+    int kept = block_best<V>([&](int j) { return o[j]; },
+                             [&](int j) { return at(j) < left ? (int)(c0 + at(j)) : -1; }, V, k, B);
+    if (kept < 0)
+        kept = best_streamed([&](int64_t i) { return make_key(src[c0 + i], (uint32_t)(c0 + i), smallest); }, left,
+                             1ull, k, B);
+    if (P > 1) {
+        kept = merge_best_parts(partial, tickets, (int)row, kept, k, B);
+        if (kept < 0) return;
     }
     for (int i = tid; i < k; i += 256) {
         const uint64_t key = i < kept ? B.keys[i] : 0ull;
@@ -200,14 +74,14 @@ __global__ __launch_bounds__(256) void topk_rows_kernel(const float* __restrict_
 }
 
 // Scores a thread holds: 16 while that leaves few workgroups (one part per
-// 4,096 scores; latency), else 32, else 64; 0 when the parts' keys would not
-// fit the merge or k is too large (the two-launch path).
+// 4,096 scores; latency), else 32, else 64; 0 when the parts would be too many
+// for the merge or k is too large (the two-launch path).
 static int topk_rows_v(int64_t rows, int64_t cols, int64_t k) {
     if (k > kBestMaxK) return 0;
     auto parts = [&](int v) { return (cols + 256 * v - 1) / (256 * v); };
     for (int v = 16; v <= 64; v <<= 1)
-        if ((v == 64 || rows * parts(v) <= 2048 || parts(2 * v) == parts(v)) && parts(v) * k <= kMergeKeys) return v;
-    return parts(64) * k <= kMergeKeys ? 64 : 0;
+        if ((v == 64 || rows * parts(v) <= 2048 || parts(2 * v) == parts(v)) && parts(v) <= kBestMaxParts) return v;
+    return 0;
 }
 
 int64_t topk_rows_parts(int64_t rows, int64_t cols, int64_t k) {

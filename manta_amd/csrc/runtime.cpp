@@ -1262,11 +1262,20 @@ int scan_topk(MantaRocm* rt, const MantaRocmCandidates* c, int dop, int order, c
     int rc = take_buffer(rt, sc, (size_t)nq * st.parts * k * 8, (void**)&partial, err);
     if (rc) return rc;
     ScanArgs a = stream_topk_args(c, q, st, k, order, out_ids, out_scores, partial, sc ? sc->tickets : rt->tickets);
-    // small k on the coalesced q8 kernel: sorted per-wave lists in registers
-    // (LDS only for merging the waves' lists)
-    if (c->format == MANTA_ROCM_Q8_ROWS && manta::q8_scan_coalesced(c->pitch) && k <= manta::kWaveListMaxK) {
+    // k <= 16 on the coalesced q8 kernel: sorted per-wave lists in registers
+    // (LDS keys only for merging the waves' lists).  Larger k: the scores of
+    // the workgroup in LDS (a word per row), selected at the end.  32 problems
+    // of 65,536 x 256: 79.2 (lists) against 87.4 us (buffered) for k = 10, 93.5
+    // against 89.4 for k = 50; one of them 12.9 against 14.7, 36.9 against 16.4.
+    const bool lists_fit = c->format == MANTA_ROCM_Q8_ROWS && manta::q8_scan_coalesced(c->pitch) &&
+                           k <= manta::kWaveListMaxK;
+    const bool buffer_fits = k <= manta::kBestMaxK && st.parts <= manta::kBestMaxParts;
+    if (lists_fit && (k <= 16 || !buffer_fits)) {
         a.wave_lists = 1;
         a.lds_keys = 256;
+    } else if (buffer_fits) {
+        a.buffered = 1;
+        a.lds_keys = st.rounds * 128;
     }
     rc = launch_scan(rt, c, dop, a, dim3((unsigned)st.parts, (unsigned)nq), (size_t)a.lds_keys * 8, err);
     if (rc) return rc;

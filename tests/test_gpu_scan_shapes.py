@@ -1,0 +1,82 @@
+"""GPU parity of the quantized-query scans over row widths and selection paths
+that the config-shaped tests do not reach: rows of any number of 16-byte
+pieces (q8) or blocks (q4), streamed a query at a time or through the
+multi-query kernels (k past 192 always takes those with 8 or more queries),
+and the buffered selection of the streaming scans (64 < k <= 192) on tied and
+clustered rows.  Bar: ids and scores bit-exact with the oracle."""
+import numpy as np
+import pytest
+
+from manta_amd import synth
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(rt, cands, want_scores, op, q, k):
+    smallest = op == "l2_distance"
+    ids, sc, _ = rt.score_topk(cands, op, rt.to_device(q), k, smallest=smallest, quantized=True)
+    want = orc.topk(want_scores, k, smallest=smallest)
+    np.testing.assert_array_equal(ids.download(), want)
+    np.testing.assert_array_equal(sc.download(), np.take_along_axis(want_scores, want, 1))
+
+
+@pytest.mark.parametrize("nq,k", [(2, 5), (3, 100), (9, 200)])
+@pytest.mark.parametrize("op", ["dot", "cosine", "l2_distance"])
+@pytest.mark.parametrize("d", [8, 24, 40, 100, 333, 520, 600, 768, 900, 1024])
+def test_q8_row_widths(rt, d, op, nq, k):
+    n = 2777
+    q = synth.normal_f16(51, d, nq, d, 1.0)
+    codes, scales = synth.q8_rows(51, 1000 + d, n, d)
+    cands = rt.bind_q8(codes, scales)
+    want = orc.score_q8(op, q, codes, scales)
+    _check(rt, cands, want, op, q, k)
+    if nq == 9:
+        got = rt.score(cands, op, rt.to_device(q), quantized=True).download()
+        np.testing.assert_array_equal(got, want)
+    cands.close()
+
+
+@pytest.mark.parametrize("nq,k", [(1, 20), (2, 150), (17, 200)])
+@pytest.mark.parametrize("op", ["dot", "cosine", "l2_distance"])
+@pytest.mark.parametrize("d", [32, 96, 160, 224, 416, 544, 800, 1024])
+def test_q4_row_widths(rt, d, op, nq, k):
+    n = 3001  # odd: with an odd number of blocks the scales end half way through a word
+    q = synth.normal_f16(52, d, nq, d, 1.0)
+    packed, scales = synth.q4_rows(52, 1000 + d, n, d)
+    cands = rt.bind_q4(packed, scales, d)
+    want = orc.score_q4(op, q, packed, scales, d)
+    _check(rt, cands, want, op, q, k)
+    if nq == 17:
+        got = rt.score(cands, op, rt.to_device(q), quantized=True).download()
+        np.testing.assert_array_equal(got, want)
+    cands.close()
+
+
+@pytest.mark.parametrize("rows", ["tied", "ascending", "clustered"])
+@pytest.mark.parametrize("fmt", ["q8", "q8_wide", "q4"])
+@pytest.mark.parametrize("n,k", [(200, 192), (5000, 65), (70000, 100), (300000, 192)])
+def test_buffered_selection(rt, fmt, rows, n, k):
+    """Rows all equal, best last, or the best ones in one thread's slots."""
+    d = 160 if fmt == "q8_wide" else 128
+    rng = np.random.default_rng(n + k)
+    q = synth.normal_f16(53, 0, 1, d, 1.0)
+    base = rng.integers(-100, 101, size=d).astype(np.int8)
+    f = np.full(n, 0.5, np.float32)
+    if rows == "ascending":
+        f = np.linspace(0.01, 1.0, n, dtype=np.float32)
+    elif rows == "clustered":
+        f = np.where(np.arange(n) % 256 == 7, np.float32(1.0) + np.arange(n, dtype=np.float32) / n, np.float32(0.25))
+    if fmt == "q4":
+        codes = np.clip(base // 15, -7, 7).astype(np.int8)
+        nib = (codes.view(np.uint8) & 15)
+        packed = np.broadcast_to(nib[0::2] | (nib[1::2] << 4), (n, d // 2)).copy()
+        scales = np.repeat(f.astype(np.float16).view(np.uint16)[:, None], d // 32, axis=1)
+        cands = rt.bind_q4(packed, scales, d)
+        want = orc.score_q4("dot", q, packed, scales, d)
+    else:
+        codes = np.broadcast_to(base, (n, d)).copy()
+        cands = rt.bind_q8(codes, f.astype(np.float32))
+        want = orc.score_q8("dot", q, codes, f.astype(np.float32))
+    _check(rt, cands, want, "dot", q, min(k, n))
+    cands.close()
