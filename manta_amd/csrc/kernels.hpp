@@ -146,7 +146,7 @@ struct MqArgs {
     const float* dnorm;         // [n]
     const float* dd;            // [n]
     int64_t n;
-    int pitch;                  // bytes per row, multiple of 32
+    int pitch;                  // bytes per row, multiple of 16 (mq_scan: at most 32 ks, the query planes' width)
     int64_t row_begin;          // rows of this pass
     int64_t row_end;
     int64_t rows_per_wg;        // rows per blockIdx.x (multiple of the chunk)
@@ -224,13 +224,13 @@ struct MqShape {
 };
 
 MqShape mq_shape(int op, int ks, int64_t nq);
-bool mq_supported_ks(int ks);
+int mq_ks(int pitch);  // smallest supported K steps (of 32 bytes) covering a row, 0 if none
 hipError_t launch_mq_scan(int op, const MqShape& sh, const MqArgs& a, dim3 grid, size_t lds, hipStream_t s);
 // q4 blocks (kernels_mq4.hip): codes = packed nibbles [n][nb*16], scales =
 // f16 [n][nb] (passed through MqArgs.scales), qhi/qlo = E16 planes in the q4
-// nibble order [nq][nb*32]; MqShape.ks holds nb.
+// nibble order [nq][ks*32]; MqShape.ks holds mq4_blocks(nb).
 MqShape mq4_shape(int op, int nb, int64_t nq);
-bool mq4_supported_nb(int nb);
+int mq4_blocks(int nb);  // smallest supported row width in blocks holding nb, 0 if none
 hipError_t launch_mq4_scan(int op, const MqShape& sh, const MqArgs& a, dim3 grid, size_t lds, hipStream_t s);
 // q8 dot with many queries (kernels_mq8.hip): 512-thread workgroups of 512
 // (ws 1) or 256 (ws 2) queries on 16x16x64 i8 MFMAs, top-k mode only; pitch

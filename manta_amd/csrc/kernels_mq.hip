@@ -33,7 +33,10 @@ namespace manta {
 
 template <int OP, int ENC, int KS, int NA, int WQ, int MODE, bool SMALL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void mq_scan_kernel(MqArgs a) {
-    constexpr int PITCH = KS * 32;           // bytes per candidate row
+    // The query planes and the LDS rows are KS*32 bytes wide; the candidate
+    // rows may be shorter (a.pitch): an LDS row then continues with bytes of
+    // the next row, which meet zero query codes.
+    constexpr int PITCH = KS * 32;
     constexpr int P = PITCH + 16;            // LDS row pitch (padding spreads banks)
     constexpr int WR = 4 / WQ;               // waves splitting the rows of a chunk (WQ: 1, 2 or 4)
     // One 32-row block per wave per chunk (WR*32 rows), two workgroups per
@@ -148,16 +151,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     // loop issues no other global loads that would have to be waited for.
     const int wave_s = __builtin_amdgcn_readfirstlane(wave);
     auto issue_chunk = [&](int64_t c0, int buf) {
-        const int8_t* base = a.codes + c0 * PITCH;
+        const int8_t* base = a.codes + c0 * a.pitch;
         const int left = (int)(r1 - c0 < CHUNK ? r1 - c0 : CHUNK);
-        const int lim = left * PITCH - 16;  // last 16 bytes inside the range
+        const int lim = left * a.pitch - 16;  // last 16 bytes inside the range
         const uint32_t t = lds_addr(tiles) + buf * TILE;
 #pragma unroll
         for (int i = 0; i < DPW; i++) {
             const int seg = wave_s * DPW + i;
             const int x = seg * 1024 + lane * 16;
             const int row = x / P;
-            const int off = row * PITCH + (x - row * P);
+            const int off = row * a.pitch + (x - row * P);
             lds_load16(base + (off < lim ? off : lim), t + seg * 1024);
         }
         const uint32_t ct = lds_addr(consts) + buf * CTILE;
@@ -831,7 +834,11 @@ MqShape mq_shape(int op, int ks, int64_t nq) {
     return s;
 }
 
-bool mq_supported_ks(int ks) { return ks == 2 || ks == 4 || ks == 8 || ks == 12 || ks == 16; }
+int mq_ks(int pitch) {
+    for (int ks : {2, 4, 8, 12, 16, 24, 32})
+        if (pitch <= 32 * ks) return ks;
+    return 0;
+}
 
 template <int OP, int ENC, int NA, int WQ, int MODE, bool SMALL, int KS>
 static hipError_t launch_mq_one(const MqArgs& a, dim3 grid, size_t lds, hipStream_t s) {
@@ -850,6 +857,8 @@ static hipError_t launch_mq_ks(const MqArgs& a, int ks, dim3 grid, size_t lds, h
         case 8: return launch_mq_one<OP, ENC, NA, WQ, MODE, SMALL, 8>(a, grid, lds, s);
         case 12: return launch_mq_one<OP, ENC, NA, WQ, MODE, SMALL, 12>(a, grid, lds, s);
         case 16: return launch_mq_one<OP, ENC, NA, WQ, MODE, SMALL, 16>(a, grid, lds, s);
+        case 24: return launch_mq_one<OP, ENC, NA, WQ, MODE, SMALL, 24>(a, grid, lds, s);
+        case 32: return launch_mq_one<OP, ENC, NA, WQ, MODE, SMALL, 32>(a, grid, lds, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -871,6 +880,7 @@ static hipError_t launch_mq_op(const MqShape& sh, const MqArgs& a, dim3 grid, si
 }
 
 hipError_t launch_mq_scan(int op, const MqShape& sh, const MqArgs& a, dim3 grid, size_t lds, hipStream_t s) {
+    if (a.pitch <= 0 || a.pitch % 16 != 0 || a.pitch > 32 * sh.ks) return hipErrorInvalidValue;
     if (op == OP_DOT) return launch_mq_op<OP_DOT, MQ_E8>(sh, a, grid, lds, s);
     if (op == OP_DOT16) return launch_mq_op<OP_DOT16, MQ_E16>(sh, a, grid, lds, s);
     if (op == OP_COSINE) return launch_mq_op<OP_COSINE, MQ_E16>(sh, a, grid, lds, s);

@@ -32,9 +32,14 @@ __device__ __forceinline__ float mq4_bound(uint64_t tk, const QConst& qc, bool s
     return smallest ? loosen_up(ts) : loosen_down(ts);
 }
 
-template <int OP, int NB, int NA, int WQ, int MODE, bool SMALL>
+// PAD: the rows have fewer than NB blocks (a.pitch / 16): an LDS row then
+// continues with bytes of the next row, the products stop at the row's last
+// block, and the query planes stay NB * 32 wide (zero past the row).
+template <int OP, int NB, int NA, int WQ, int MODE, bool SMALL, bool PAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void mq_q4_kernel(MqArgs a) {
-    constexpr int PITCH = NB * 16;            // packed bytes per candidate row
+    const int nb = PAD ? a.pitch / 16 : NB;   // blocks per row
+    const int gpitch = PAD ? a.pitch : NB * 16;  // packed bytes per candidate row
+    constexpr int PITCH = NB * 16;
     constexpr int D = NB * 32;                // elements per row (query plane width)
     constexpr int P = PITCH + 16;             // LDS row pitch
     constexpr int WR = 4 / WQ;                // waves splitting the rows of a chunk
@@ -126,21 +131,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     const uint8_t* sc_bytes = (const uint8_t*)a.scales;
     const float* rowc_src = OP == OP_COSINE ? a.dnorm : a.dd;
     auto issue_chunk = [&](int64_t c0, int buf) {
-        const int8_t* base = a.codes + c0 * PITCH;
+        const int8_t* base = a.codes + c0 * gpitch;
         const int left = (int)(r1 - c0 < CHUNK ? r1 - c0 : CHUNK);
-        const int lim = left * PITCH - 16;
+        const int lim = left * gpitch - 16;
         const uint32_t t = lds_addr(tiles) + buf * TILE;
 #pragma unroll
         for (int i = 0; i < DPW; i++) {
             const int seg = wave_s * DPW + i;
             const int x = seg * 1024 + lane * 16;
             const int row = x / P;
-            const int off = row * PITCH + (x - row * P);
+            const int off = row * gpitch + (x - row * P);
             lds_load16(base + (off < lim ? off : lim), t + seg * 1024);
         }
         const uint32_t ct = lds_addr(consts) + buf * CTILE;
-        const uint8_t* sbase = sc_bytes + c0 * (NB * 2);
-        const int slim = left * NB * 2 - 4;
+        const uint8_t* sbase = sc_bytes + c0 * (nb * 2);
+        // the last whole word of the range's scales (an odd count ends half
+        // way through it; the scales' allocation is padded to a word)
+        const int slim = (left * nb * 2 - 1) & ~3;
 #pragma unroll
         for (int i = 0; i < CPW; i++) {
             const int cs = wave_s * CPW + i;  // segments past SCSEG + RCSEG are filler
@@ -166,7 +173,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     // b+2's B fragment -- hence its MFMA -- comes after it.
     auto multiply = [&](const uint8_t* tile, const uint8_t* ctile, float (&dotf)[NA][QPL]) {
         const uint8_t* bp = tile + (wr * 32 + (lane & 31)) * P + half * 8;
-        const uint16_t* sp = (const uint16_t*)ctile + (wr * 32 + (lane & 31)) * NB;
+        const uint16_t* sp = (const uint16_t*)ctile + (wr * 32 + (lane & 31)) * nb;
         auto widen = [&](int b) {
             const uint2 nb2 = *(const uint2*)(bp + b * 16);
             v4i bf = {(int)((nb2.x << 4) & 0xF0F0F0F0u), (int)(nb2.x & 0xF0F0F0F0u),
@@ -186,6 +193,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
         }
 #pragma unroll
         for (int b = 0; b < NB; b++) {
+            if (PAD && b >= nb) break;
             v16i acc[NA];
 #pragma unroll
             for (int na = 0; na < NA; na++) acc[na] = accn[na];
@@ -391,13 +399,23 @@ MqShape mq4_shape(int op, int nb, int64_t nq) {
     return s;
 }
 
-bool mq4_supported_nb(int nb) { return nb == 1 || nb == 2 || nb == 4 || nb == 8 || nb == 12 || nb == 16; }
+int mq4_blocks(int nb) {
+    for (int b : {1, 2, 4, 8, 12, 16, 24, 32})
+        if (nb <= b) return b;
+    return 0;
+}
 
 template <int OP, int NA, int WQ, int MODE, bool SMALL, int NB>
 static hipError_t launch_mq4_one(const MqArgs& a, dim3 grid, size_t lds, hipStream_t s) {
     if constexpr (mq4_valid(NA, WQ, NB)) {
-        hipLaunchKernelGGL((mq_q4_kernel<OP, NB, NA, WQ, MODE, SMALL>), grid, dim3(256), lds, s, a);
-        return hipGetLastError();
+        if (a.pitch == 16 * NB) {
+            hipLaunchKernelGGL((mq_q4_kernel<OP, NB, NA, WQ, MODE, SMALL, false>), grid, dim3(256), lds, s, a);
+            return hipGetLastError();
+        }
+        if constexpr (NB > 2) {
+            hipLaunchKernelGGL((mq_q4_kernel<OP, NB, NA, WQ, MODE, SMALL, true>), grid, dim3(256), lds, s, a);
+            return hipGetLastError();
+        }
     }
     return hipErrorInvalidValue;
 }
@@ -411,6 +429,8 @@ static hipError_t launch_mq4_nb(const MqArgs& a, int nb, dim3 grid, size_t lds, 
         case 8: return launch_mq4_one<OP, NA, WQ, MODE, SMALL, 8>(a, grid, lds, s);
         case 12: return launch_mq4_one<OP, NA, WQ, MODE, SMALL, 12>(a, grid, lds, s);
         case 16: return launch_mq4_one<OP, NA, WQ, MODE, SMALL, 16>(a, grid, lds, s);
+        case 24: return launch_mq4_one<OP, NA, WQ, MODE, SMALL, 24>(a, grid, lds, s);
+        case 32: return launch_mq4_one<OP, NA, WQ, MODE, SMALL, 32>(a, grid, lds, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -432,6 +452,7 @@ static hipError_t launch_mq4_op(const MqShape& sh, const MqArgs& a, dim3 grid, s
 }
 
 hipError_t launch_mq4_scan(int op, const MqShape& sh, const MqArgs& a, dim3 grid, size_t lds, hipStream_t s) {
+    if (a.pitch <= 0 || a.pitch % 16 != 0 || a.pitch > 16 * sh.ks) return hipErrorInvalidValue;
     if (op == OP_DOT) return launch_mq4_op<OP_DOT>(sh, a, grid, lds, s);
     if (op == OP_COSINE) return launch_mq4_op<OP_COSINE>(sh, a, grid, lds, s);
     return launch_mq4_op<OP_L2>(sh, a, grid, lds, s);

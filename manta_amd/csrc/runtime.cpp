@@ -709,7 +709,8 @@ int manta_rocm_bind_q4_blocks(MantaRocm* rt, const uint8_t* packed, const uint16
     c->nb = nb;
     c->bytes = (size_t)rows * (pitch + nb * 2 + 16);
     hipError_t e = hipMalloc(&c->codes, (size_t)rows * pitch);
-    if (e == hipSuccess) e = hipMalloc(&c->scales, (size_t)rows * nb * 2);
+    // (whole words: the multi-query kernel loads scales 4 bytes at a time)
+    if (e == hipSuccess) e = hipMalloc(&c->scales, align_up((size_t)rows * nb * 2, 4));
     if (e == hipSuccess) e = hipMalloc((void**)&c->dnorm, (size_t)rows * 4);
     if (e == hipSuccess) e = hipMalloc((void**)&c->dd, (size_t)rows * 4);
     if (e == hipSuccess) e = hipMalloc((void**)&c->sqd, (size_t)rows * 8);
@@ -977,9 +978,22 @@ void ensure_q4_shadow(MantaRocm* rt, const MantaRocmCandidates* c) {
     rt->stats.candidate_bytes += extra;
 }
 
+// Little work: the passes' launches (encoding, then a scan and a select each)
+// would cost more than one streaming launch that reads the cached rows once
+// per query.  Whole reference calls, passes against streaming: q8, 8 queries x
+// 80,000 x 384 67 / 57 us, 32 x 20,000 x 256 64 / 50; past the line 8 x 50,000 x
+// 768 and 8 x 200,000 x 128 are even, 100 x 4,000 x 1,000 streams in 168 against
+// 103.  Up to 4,096 q8 rows the passes are one, and 512 x 1,200 x 256 takes 52
+// against 63.  (k past kBestMaxK streams through the reservoir: the passes.)
+bool stream_is_faster(const MantaRocmCandidates* c, int64_t nq, int64_t k) {
+    const double limit = c->format == MANTA_ROCM_Q8_ROWS && c->n <= 4096 ? 3e8 : 5e8;
+    return k <= manta::kBestMaxK && (double)nq * (double)c->n * (double)(c->d + 256) < limit;
+}
+
 MqPlan mq_plan(const MantaRocmCandidates* c, int dop, int64_t nq, int64_t k, bool topk) {
     MqPlan p;
     if (c->sets != 1 || nq < 8) return p;
+    if (topk && stream_is_faster(c, nq, k)) return p;
     // the 16x16x64 kernel: 512-query groups, or 256 with the rows of a chunk
     // split over two wave groups
     const int ws8 = nq >= 512 ? 1 : 2;
@@ -988,8 +1002,9 @@ MqPlan mq_plan(const MantaRocmCandidates* c, int dop, int64_t nq, int64_t k, boo
             mq8_fits(c->pitch, k)) {
             p.sh = manta::mq8_shape(c->pitch, ws8, false);
         } else {
-            if (c->pitch % 32 != 0 || !manta::mq_supported_ks(c->pitch / 32)) return p;
-            p.sh = manta::mq_shape(dop, c->pitch / 32, nq);
+            const int ks = manta::mq_ks(c->pitch);
+            if (!ks) return p;
+            p.sh = manta::mq_shape(dop, ks, nq);
         }
     } else {
         p.q4 = true;
@@ -997,8 +1012,9 @@ MqPlan mq_plan(const MantaRocmCandidates* c, int dop, int64_t nq, int64_t k, boo
             p.shadow = true;
             p.sh = manta::mq8_shape(c->shadow_pitch, ws8, true);
         } else {
-            if (!manta::mq4_supported_nb(c->nb)) return p;
-            p.sh = manta::mq4_shape(dop, c->nb, nq);
+            const int blocks = manta::mq4_blocks(c->nb);
+            if (!blocks) return p;
+            p.sh = manta::mq4_shape(dop, blocks, nq);
         }
     }
     p.groups = (int)((nq + p.sh.qg - 1) / p.sh.qg);
@@ -1089,10 +1105,10 @@ hipError_t launch_mq_pass(const MqPlan& p, int dop, const manta::MqArgs& a, int 
 int run_mq(MantaRocm* rt, const MantaRocmCandidates* c, int dop, int order, const uint16_t* q, int64_t nq,
            int64_t k, const MqPlan& p, float* out_scores, int32_t* out_ids, float* out_topk_scores,
            char** err, bool any_order = false) {
-    // query planes: E8 codes or E16 digits, one row per query, as wide as a
-    // q8 row (pitch) or a q4 row in elements (d); the shadow scan's E8
-    // codes are as wide as a shadow row, its E16 planes [nq][d]
-    const int width = p.shadow ? c->shadow_pitch : (p.q4 ? (int)c->d : c->pitch);
+    // query planes: E8 codes or E16 digits, one row per query, as wide as the
+    // kernel's rows in elements (at least d, zero padded); the shadow scan's
+    // E8 codes are as wide as a shadow row, its E16 planes [nq][d]
+    const int width = p.shadow ? c->shadow_pitch : (p.sh.kind == 1 ? c->pitch : 32 * p.sh.ks);
     const size_t plane = (size_t)nq * width;
     const bool topk = out_scores == nullptr;
     const size_t regions = topk ? (size_t)nq * p.rmax * p.rc : 0;
