@@ -129,8 +129,10 @@ struct RefArgs {
 // keys [nq][kp]: the reference key of each candidate (ref_rescore), then
 // the finish over them.
 hipError_t launch_ref_rescore(const RefArgs& a, uint64_t* keys, hipStream_t s);
+// Score matrix out [nq][n] (the fields up to op).
+hipError_t launch_ref_scores(const RefArgs& a, float* out, hipStream_t s);
 hipError_t launch_ref_finish(const RefArgs& a, const uint64_t* keys, hipStream_t s);
-// Reference scores of every row (score matrix: a.out_scores, grid
+// Reference scores of every row, lane = row (score matrix: a.out_scores, grid
 // (parts, nq)) or top-k with the streaming reservoir and last-workgroup merge
 // (ScanArgs as for the streaming scans; grid (parts, R), each blockIdx.y
 // taking every R-th query).  redo / redo_tau (may be null: every query, no

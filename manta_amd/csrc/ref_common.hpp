@@ -112,6 +112,7 @@ __device__ inline double div_rn(double a, double b) {
 // The reference's f64 norm term sqrt(sum x^2), summed in column order.
 __device__ inline double ref_sqrt_norm(const float* x, int d) {
     double s = 0.0;
+#pragma unroll 8
     for (int c = 0; c < d; c++) s = __fma_rn((double)x[c], (double)x[c], s);
     return sqrt_rn(s);
 }

@@ -1229,14 +1229,35 @@ int manta_rocm_score(MantaRocm* rt, const MantaRocmCandidates* c, int op, const 
     const ScoreOp so = parse_op(c, op);
     const int64_t tiles = (c->n + 255) / 256;
     if (!so.quant) {
-        // the reference arithmetic for every (query, row)
-        ScanArgs a = scan_args(c, q);
-        a.rounds = (int)std::max<int64_t>(1, std::min<int64_t>(16, tiles * nq / 2048));
-        a.out_scores = out;
-        const int64_t parts = (tiles + a.rounds - 1) / a.rounds;
-        LAUNCH_TRY(manta::launch_ref_scan(c->format == MANTA_ROCM_Q8_ROWS ? 8 : 4, so.ref, a, (int)nq, c->sqd,
-                                          nullptr, nullptr, dim3((unsigned)parts, (unsigned)nq), 0, rt->stream),
-                   "ref_scan");
+        // the reference arithmetic for every (query, row).  q4 rows for one or
+        // two queries: straight from memory, lane = row (one query x 300,000,
+        // d 256: 17.9 us, the tiles 31; two x 1,000,000, d 128: 38.9 and 53);
+        // otherwise, and for few rows, tiles of rows and queries through LDS
+        // (one x 60,000, d 384: 9.3 and 11; four x 5,000: 36.9 and 12.4)
+        const int fmt = c->format == MANTA_ROCM_Q8_ROWS ? 8 : 4;
+        if (fmt == 4 && (nq <= 2 || c->sets > 1) && c->n * nq >= 32768) {
+            ScanArgs a = scan_args(c, q);
+            a.rounds = (int)std::max<int64_t>(1, std::min<int64_t>(16, tiles * nq / 2048));
+            a.out_scores = out;
+            const int64_t parts = (tiles + a.rounds - 1) / a.rounds;
+            LAUNCH_TRY(manta::launch_ref_scan(fmt, so.ref, a, (int)nq, c->sqd, nullptr, nullptr,
+                                              dim3((unsigned)parts, (unsigned)nq), 0, rt->stream),
+                       "ref_scan");
+            return MANTA_ROCM_OK;
+        }
+        manta::RefArgs ra{};
+        ra.fmt = fmt;
+        ra.codes = c->codes;
+        ra.scales = c->scales;
+        ra.sqd = c->sqd;
+        ra.n = c->n;
+        ra.pitch = c->pitch;
+        ra.d = (int)c->d;
+        ra.set_stride = c->sets == 1 ? 0 : c->n;
+        ra.queries = q;
+        ra.nq = (int)nq;
+        ra.op = so.ref;
+        LAUNCH_TRY(manta::launch_ref_scores(ra, out, rt->stream), "ref_scores");
         return MANTA_ROCM_OK;
     }
     const MqPlan plan = mq_plan(c, so.scan, nq, 0, false);
