@@ -685,15 +685,18 @@ __global__ __launch_bounds__(256) void q8_scan_generic_kernel(ScanArgs a) {
     const int wg_rows = left < (int64_t)a.rounds * 256 ? (int)left : a.rounds * 256;
     const __amdgpu_buffer_rsrc_t rs =
         byte_buffer(a.codes + (set_row0 + wg_row0) * a.pitch, (uint32_t)wg_rows * a.pitch);
-    // past the buffer, whatever row is added: such loads touch no memory
-    constexpr int kFar = 0x40000000;
-    const int voff = act ? (wave * 64 + g) * a.pitch + p * 16 : kFar;
+    // past the buffer, whatever row is added: such loads touch no memory.  (The
+    // whole offset is the lanes': the scalar offset has no part in the bounds
+    // check.  Unsigned, as the check is: two of them do not wrap.)
+    constexpr uint32_t kFar = 0x7ffffff0u;
+    const uint32_t voff = act ? (uint32_t)((wave * 64 + g) * a.pitch + p * 16) : kFar;
     v4i w[B], wn[B];
     auto load = [&](v4i (&dw)[B], int r, int s0) {
 #pragma unroll
         for (int j = 0; j < B; j++) {
             const bool in = s0 + j < steps;  // the same for the whole wave
-            dw[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, in ? (r * 256 + (s0 + j) * rpl) * a.pitch : kFar, 2);
+            const uint32_t off = in ? (uint32_t)((r * 256 + (s0 + j) * rpl) * a.pitch) : kFar;
+            dw[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff + off, 0, 2);
         }
     };
     load(w, 0, 0);
@@ -799,9 +802,10 @@ __global__ __launch_bounds__(256) void q4_scan_kernel(ScanArgs a) {
     const __amdgpu_buffer_rsrc_t ss =
         byte_buffer((const uint16_t*)a.scales + (set_row0 + wg_row0) * nb, (uint32_t)wg_rows * nb * 2);
     // past every buffer, whatever row is added: such loads touch no memory
-    constexpr int kFar = 0x40000000;
-    const int voff = act ? (wave * 64 + g) * a.pitch + p * 16 : kFar;
-    const int soff = act ? ((wave * 64 + g) * nb + p) * 2 : kFar;
+    // (the whole offset is the lanes', as above)
+    constexpr uint32_t kFar = 0x7ffffff0u;
+    const uint32_t voff = act ? (uint32_t)((wave * 64 + g) * a.pitch + p * 16) : kFar;
+    const uint32_t soff = act ? (uint32_t)(((wave * 64 + g) * nb + p) * 2) : kFar;
     v4i w[B], wn[B];
     uint16_t sc[B], scn[B];
     auto load = [&](v4i (&dw)[B], uint16_t (&ds)[B], int r, int s0) {
@@ -809,8 +813,8 @@ __global__ __launch_bounds__(256) void q4_scan_kernel(ScanArgs a) {
         for (int j = 0; j < B; j++) {
             const int row = r * 256 + (s0 + j) * rpl;
             const bool in = s0 + j < steps;  // the same for the whole wave
-            dw[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, in ? row * a.pitch : kFar, 2);
-            ds[j] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(ss, soff, in ? row * nb * 2 : kFar, 2);
+            dw[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff + (in ? (uint32_t)(row * a.pitch) : kFar), 0, 2);
+            ds[j] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(ss, soff + (in ? (uint32_t)(row * nb * 2) : kFar), 0, 2);
         }
     };
     load(w, sc, 0, 0);
