@@ -266,7 +266,7 @@ __device__ __forceinline__ void emit_round(const ScanArgs& a, float score, bool 
 // a barrier or an atomic; the k best of them, and of the query's parts, by a
 // floor and ranks.  Against the reservoir (compactions between rounds, the
 // last workgroup streaming every part key through it): one q4 query, 1,048,576
-// rows, k = 108, 159 -> 57 us.
+// rows, k = 108, 159 -> 65 us.
 __device__ __forceinline__ void finish_buffered(const ScanArgs& a, const uint64_t* buf, int qi) {
     __shared__ BestShared B;
     const uint32_t* slots = (const uint32_t*)buf;  // (rows past n: 0)
@@ -780,7 +780,7 @@ __global__ __launch_bounds__(256) void q8_scan_generic_kernel(ScanArgs a) {
 // pitch nb | 1: 64 rows on distinct banks).  Loads are 8 instructions ahead,
 // across rounds too.  The read of the rows bounds it: one query against
 // 1,048,576 x 384 rows took 167 us with a row per lane (16 bytes out of every
-// 192 per load), 57 this way with the selection (226 MB: 46 us at the copy
+// 192 per load), 65 this way with the selection (226 MB: 46 us at the copy
 // rate).
 template <int OP>
 __global__ __launch_bounds__(256) void q4_scan_kernel(ScanArgs a) {
