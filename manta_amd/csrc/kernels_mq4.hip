@@ -19,6 +19,7 @@
 // Chunks, passes, regions, compaction and the select are those of the q8
 // multi-query path (kernels_mq.hip).
 #include "mq_common.hpp"
+#include "mq_plan.hpp"
 
 namespace manta {
 
@@ -145,9 +146,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
         }
         const uint32_t ct = lds_addr(consts) + buf * CTILE;
         const uint8_t* sbase = sc_bytes + c0 * (nb * 2);
-        // the last whole word of the range's scales (an odd count ends half
-        // way through it; the scales' allocation is padded to a word)
-        const int slim = (left * nb * 2 - 1) & ~3;
+        const int slim = mq4_scale_limit(left, nb);
 #pragma unroll
         for (int i = 0; i < CPW; i++) {
             const int cs = wave_s * CPW + i;  // segments past SCSEG + RCSEG are filler
@@ -453,6 +452,8 @@ static hipError_t launch_mq4_op(const MqShape& sh, const MqArgs& a, dim3 grid, s
 
 hipError_t launch_mq4_scan(int op, const MqShape& sh, const MqArgs& a, dim3 grid, size_t lds, hipStream_t s) {
     if (a.pitch <= 0 || a.pitch % 16 != 0 || a.pitch > 16 * sh.ks) return hipErrorInvalidValue;
+    // (the scales' word copies: mq4_scale_limit)
+    if (a.row_begin % 2 != 0 || a.rows_per_wg % sh.chunk != 0) return hipErrorInvalidValue;
     if (op == OP_DOT) return launch_mq4_op<OP_DOT>(sh, a, grid, lds, s);
     if (op == OP_COSINE) return launch_mq4_op<OP_COSINE>(sh, a, grid, lds, s);
     return launch_mq4_op<OP_L2>(sh, a, grid, lds, s);

@@ -27,6 +27,7 @@
 
 #include "device_common.hpp"
 #include "kernels.hpp"
+#include "mq_plan.hpp"
 #include "pack.hpp"
 #include "runtime_internal.hpp"
 
@@ -888,16 +889,8 @@ namespace {
 
 // Multi-query plan: many queries against one shared q8 matrix go to the
 // matrix-core kernels (kernels_mq.hip); everything else streams one query per
-// workgroup.  Top-k runs in passes over growing row prefixes: pass 0 keeps
-// every key of its rows, and each later pass starts from the k-th best key
-// of all earlier rows, so only a few times k keys per query survive a pass.
-struct MqPass {
-    int64_t begin = 0;
-    int64_t end = 0;
-    int64_t rows_per_wg = 0;
-    int R = 0;
-    int select_threads = 256;
-};
+// workgroup.  Passes: mq_plan.hpp.
+using manta::MqPass;
 
 struct MqPlan {
     bool use = false;
@@ -913,24 +906,10 @@ struct MqPlan {
 
 constexpr int kMqWorkgroups = 512;     // two 256-thread workgroups per CU of a 256-CU MI355X
 constexpr int kMq8Workgroups = 256;    // one 512-thread workgroup per CU
-constexpr int64_t kMqSelectKeys = 16384;  // LDS keys of the select kernel
-
-MqPass mq_pass(int64_t begin, int64_t end, int chunk, int groups, int64_t max_rows_per_wg, int wgs) {
-    MqPass p;
-    p.begin = begin;
-    p.end = end;
-    const int64_t chunks = (end - begin + chunk - 1) / chunk;
-    int64_t R = std::max<int64_t>(1, std::min<int64_t>(chunks, std::max(1, wgs / groups)));
-    int64_t cpw = (chunks + R - 1) / R;
-    if (max_rows_per_wg > 0) cpw = std::max<int64_t>(1, std::min<int64_t>(cpw, max_rows_per_wg / chunk));
-    p.rows_per_wg = cpw * chunk;
-    p.R = (int)((chunks + cpw - 1) / cpw);
-    return p;
-}
 
 // Region capacity of the 512-query kernel for k; its free chunk tile must
 // hold a region's pairs and keys when it compacts one.
-int mq8_rc(int64_t k) { return (int)(((2 * k + 2 * 64 + 64) + 63) / 64 * 64); }
+int mq8_rc(int64_t k) { return manta::mq_region_keys(k, 64); }
 
 bool mq8_fits(int pitch, int64_t k) {
     return manta::mq8_supported(pitch) && (size_t)mq8_rc(k) * 16 <= (size_t)manta::mq8_shape(pitch, 1, false).tile;
@@ -1022,71 +1001,23 @@ MqPlan mq_plan(const MantaRocmCandidates* c, int dop, int64_t nq, int64_t k, boo
     const int chunk = p.sh.chunk;
     const int wgs = p.sh.kind == 1 ? kMq8Workgroups : kMqWorkgroups;
     if (!topk) {
-        p.passes.push_back(mq_pass(0, c->n, chunk, p.groups, 0, wgs));
+        p.passes.push_back(manta::mq_pass(0, c->n, chunk, p.groups, 0, wgs));
         p.rmax = p.passes[0].R;
         p.lds = (size_t)p.sh.tile_bytes;
         p.use = true;
         return p;
     }
-    // region: the best k after a compaction plus one chunk of appends, with
-    // slack so a compaction frees at least k slots (the 512-query kernel
-    // needs rc >= k + 2.5 chunks: true for its chunks of 64 or 128 rows)
-    p.rc = (int)(((2 * k + 2 * chunk + 64) + 63) / 64 * 64);
+    p.rc = manta::mq_region_keys(k, chunk);
     p.lds = (size_t)p.sh.tile_bytes +
             (p.sh.kind == 0 && (size_t)p.rc * 8 > (size_t)p.sh.tile ? (size_t)p.rc * 8 : 0);
-    // pass 0: everything is kept, so a workgroup takes at most rc - 2*chunk rows
-    int64_t s = std::min<int64_t>(c->n, std::max<int64_t>(8 * k, 4096));
-    p.passes.push_back(mq_pass(0, s, chunk, p.groups, p.rc - 2 * chunk, wgs));
-    p.passes.back().select_threads = manta::mq_select_threads(s);
-    // shadow pairs are rescored by the select: 512 threads keep many row
-    // loads in flight within the register budget
-    if (p.shadow) p.passes.back().select_threads = 512;
-    if (s < c->n) {
-        // later passes grow the prefix by g: about k*g keys per query reach
-        // the select.  Fewest passes the select's buffer allows, then the
-        // smallest g that still needs no more of them.
-        const double span = (double)c->n / (double)s;
-        const double gmax = std::max(4.0, (double)kMqSelectKeys / (double)k);
-        int npass = std::max(1, (int)std::ceil(std::log(span) / std::log(gmax) - 1e-9));
-        // the 512-query kernel appends about k*(g-1) pairs per query and
-        // pass, each an exact test and an LDS atomic in the scan: keep g
-        // near 4.5 (measured on 1024 queries over 1024x the first pass's
-        // rows: 5 passes beat 3 by 4% of the step, 6 and 7 lose to 5 on the
-        // selects)
-        if (p.sh.kind == 1 && !p.shadow)
-            npass = std::max(npass, (int)std::ceil(std::log(span) / std::log(4.5) - 1e-9));
-        // shadow pairs: every pair the select keeps is rescored from a random
-        // row, so fewer, larger passes win as long as a pass's pairs (about
-        // 4*k*g with the margins) fit the 512-thread select's 8K-key buffer,
-        // which is what lets it prune before rescoring
-        if (p.shadow) {
-            const double gs = std::max(4.0, (8192.0 - (double)k) / (4.0 * (double)k));
-            npass = std::max(1, (int)std::ceil(std::log(span) / std::log(gs) - 1e-9));
-        }
-        double g = std::pow(span, 1.0 / npass);
-        // ... except its first growth pass, which grows the prefix by 16: over
-        // so few rows the extra appends cost less than a pass and a select of
-        // their own (1024 queries over 4M rows: 4,096 rows, then x16 and
-        // three times x4 -- five passes instead of six -- measured 1,422 ->
-        // 1,400 us a call; x8 gained nothing, x64 lost 35 us)
-        double g0 = g;
-        const double gfirst = std::min(16.0, gmax);
-        if (p.sh.kind == 1 && !p.shadow && span > gfirst * 4.5) {
-            const double rest = span / gfirst;
-            npass = 1 + (int)std::ceil(std::log(rest) / std::log(4.5) - 1e-9);
-            g0 = gfirst;
-            g = std::pow(rest, 1.0 / (npass - 1));
-        }
-        for (int i = 0; i < npass; i++) {
-            const double gi = i == 0 ? g0 : g;
-            const int64_t e = i + 1 == npass ? c->n : std::min<int64_t>(c->n, (int64_t)std::ceil(s * gi));
-            if (e <= s) continue;
-            p.passes.push_back(mq_pass(s, e, chunk, p.groups, 0, wgs));
-            // (shadow pairs: the margins let a few times more through)
-            p.passes.back().select_threads =
-                p.shadow ? 512 : manta::mq_select_threads(k + (int64_t)(k * (gi - 1.0) * 1.5));
-            s = e;
-        }
+    p.passes = manta::mq_topk_passes(c->n, k, chunk, p.groups, wgs, p.sh.kind == 1, p.shadow);
+    for (MqPass& ps : p.passes) {
+        // about k*(g-1) keys pass the threshold of a growth pass, all rows of
+        // the first.  Shadow pairs are rescored by the select: 512 threads
+        // keep many row loads in flight within the register budget (and the
+        // margins let a few times more through).
+        const int64_t keys = ps.begin == 0 ? ps.end : k + (int64_t)(k * (ps.grow - 1.0) * 1.5);
+        ps.select_threads = p.shadow ? 512 : manta::mq_select_threads(keys);
     }
     for (const MqPass& ps : p.passes) p.rmax = std::max(p.rmax, ps.R);
     // the kernels index regions with 32-bit offsets
