@@ -30,6 +30,7 @@
 #include "mq_plan.hpp"
 #include "pack.hpp"
 #include "runtime_internal.hpp"
+#include "stream_plan.hpp"
 
 using manta::QConst;
 using manta::ScanArgs;
@@ -811,22 +812,6 @@ int check_score_args(const MantaRocmCandidates* c, int op_in, const void* q, int
     return MANTA_ROCM_OK;
 }
 
-// Rounds of 256 rows per scan workgroup, for about `wgs` workgroups in all,
-// so each streams a long contiguous range and the per-workgroup prologue and
-// top-k publication are paid rarely.  The fused top-k takes one workgroup
-// per CU (C0's 32 problems: 82.3 us a launch against 85.1 with two per CU,
-// 97.6 with one per two CUs and 99.2 with 1.25 per CU); the score matrix
-// keeps two per CU.
-int choose_rounds(int64_t tiles, int64_t nq, int64_t wgs) {
-    int64_t r = (tiles * nq + wgs - 1) / wgs;
-    // small calls are latency-bound: two rounds halve the parts the last
-    // workgroup merges (one 65536 x 256 query, with the lists filled and
-    // merged by rank: 13.3 us a call against 15.8 with one round and 14.1
-    // with four)
-    if (r < 2 && tiles >= 4) r = 2;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(64, r));
-}
-
 // Launch shape of a streaming top-k (one query per blockIdx.y): `parts`
 // workgroups of `rounds` x 256 rows per query, and the LDS reservoir.  A
 // reservoir that holds every row of the workgroup needs no compaction (and
@@ -915,6 +900,12 @@ bool mq8_fits(int pitch, int64_t k) {
     return manta::mq8_supported(pitch) && (size_t)mq8_rc(k) * 16 <= (size_t)manta::mq8_shape(pitch, 1, false).tile;
 }
 
+// A top-k that streams one query per workgroup although the passes could take
+// it (k past kBestMaxK streams through the reservoir: the passes).
+bool stream_is_faster(const MantaRocmCandidates* c, int64_t nq, int64_t k) {
+    return k <= manta::kBestMaxK && manta::stream_is_faster(c->format == MANTA_ROCM_Q8_ROWS, c->n, c->d, nq);
+}
+
 // q4 cosine / dot top-k with at least 256 queries goes through the int8
 // shadow (built on first use).
 bool q4_shadow_wanted(const MantaRocmCandidates* c, int dop, int64_t nq, int64_t k) {
@@ -955,18 +946,6 @@ void ensure_q4_shadow(MantaRocm* rt, const MantaRocmCandidates* c) {
     const size_t extra = (size_t)n * sp + (size_t)n * 8 + sizeof(manta::ShadowInfo);
     c->bytes += extra;
     rt->stats.candidate_bytes += extra;
-}
-
-// Little work: the passes' launches (encoding, then a scan and a select each)
-// would cost more than one streaming launch that reads the cached rows once
-// per query.  Whole reference calls, passes against streaming: q8, 8 queries x
-// 80,000 x 384 67 / 57 us, 32 x 20,000 x 256 64 / 50; past the line 8 x 50,000 x
-// 768 and 8 x 200,000 x 128 are even, 100 x 4,000 x 1,000 streams in 168 against
-// 103.  Up to 4,096 q8 rows the passes are one, and 512 x 1,200 x 256 takes 52
-// against 63.  (k past kBestMaxK streams through the reservoir: the passes.)
-bool stream_is_faster(const MantaRocmCandidates* c, int64_t nq, int64_t k) {
-    const double limit = c->format == MANTA_ROCM_Q8_ROWS && c->n <= 4096 ? 3e8 : 5e8;
-    return k <= manta::kBestMaxK && (double)nq * (double)c->n * (double)(c->d + 256) < limit;
 }
 
 MqPlan mq_plan(const MantaRocmCandidates* c, int dop, int64_t nq, int64_t k, bool topk) {
@@ -1194,7 +1173,7 @@ int manta_rocm_score(MantaRocm* rt, const MantaRocmCandidates* c, int op, const 
     const MqPlan plan = mq_plan(c, so.scan, nq, 0, false);
     if (plan.use) return run_mq(rt, c, so.scan, MANTA_ROCM_LARGEST, q, nq, 0, plan, out, nullptr, nullptr, err);
     ScanArgs a = scan_args(c, q);
-    a.rounds = choose_rounds(tiles, nq, 512);
+    a.rounds = manta::choose_rounds(tiles, nq, 512);
     a.out_scores = out;
     const int64_t parts = (tiles + a.rounds - 1) / a.rounds;
     return launch_scan(rt, c, so.scan, a, dim3((unsigned)parts, (unsigned)nq), 0, err);
@@ -1225,7 +1204,7 @@ int scan_topk(MantaRocm* rt, const MantaRocmCandidates* c, int dop, int order, c
                        "q8_rescore");
         return MANTA_ROCM_OK;
     }
-    StreamTopk st = stream_topk_shape(c, nq, k, choose_rounds((c->n + 255) / 256, nq, rt->cus));
+    StreamTopk st = stream_topk_shape(c, nq, k, manta::choose_rounds((c->n + 255) / 256, nq, rt->cus));
     uint64_t* partial = nullptr;
     int rc = take_buffer(rt, sc, (size_t)nq * st.parts * k * 8, (void**)&partial, err);
     if (rc) return rc;
