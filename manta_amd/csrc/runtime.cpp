@@ -910,7 +910,8 @@ bool stream_is_faster(const MantaRocmCandidates* c, int64_t nq, int64_t k) {
 // shadow (built on first use).
 bool q4_shadow_wanted(const MantaRocmCandidates* c, int dop, int64_t nq, int64_t k) {
     return c->format == MANTA_ROCM_Q4_BLOCKS && c->sets == 1 && (dop == manta::OP_COSINE || dop == manta::OP_DOT) &&
-           nq >= 256 && c->d <= 384 && c->scales_finite && mq8_fits((int)align_up((size_t)c->d, 128), k);
+           nq >= 256 && c->d <= 384 && c->scales_finite && mq8_fits((int)align_up((size_t)c->d, 128), k) &&
+           !stream_is_faster(c, nq, k);
 }
 
 // Build the int8 shadow of a q4 matrix on its first many-query top-k call

@@ -182,3 +182,21 @@ def test_repeated_calls_start_afresh(rt):
         cands = rt.bind_q8(codes, scales)
         _check(rt, cands, "l2_distance", q, 100, True, orc.score_q8("l2_distance", q, codes, scales), passes=2)
         cands.close()
+
+
+def test_small_calls_build_no_shadow(rt):
+    """A q4 call of many queries that streams leaves the bound matrix as it
+    is; the first one past the line builds the shadow and keeps it."""
+    d, k = 64, 10
+    q = synth.normal_f16(77, 0, 256, d, 1.0, normalize=True)
+    for n, built in ((3000, False), (12000, True)):
+        packed, scales = synth.q4_rows(77, 1, n, d, normalize=True)
+        cands = rt.bind_q4(packed, scales, d)
+        before = rt.stats()["candidate_bytes"]
+        ids, sc = _topk(rt, cands, "cosine", q, k, False)
+        want_s = orc.score_q4("cosine", q, packed, scales, d)
+        want = orc.topk(want_s, k)
+        np.testing.assert_array_equal(ids, want)
+        np.testing.assert_array_equal(sc, np.take_along_axis(want_s, want, 1))
+        assert (rt.stats()["candidate_bytes"] > before) == built, n
+        cands.close()
