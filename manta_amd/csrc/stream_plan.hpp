@@ -28,14 +28,29 @@ inline int choose_rounds(int64_t tiles, int64_t nq, int64_t wgs) {
 
 // Little work: the multi-query passes' launches (encoding, then a scan and a
 // select each) would cost more than one streaming launch that reads the cached
-// rows once per query.  Whole reference calls, passes against streaming: q8, 8 queries x
-// 80,000 x 384 67 / 57 us, 32 x 20,000 x 256 64 / 50; past the line 8 x 50,000 x
-// 768 and 8 x 200,000 x 128 are even, 100 x 4,000 x 1,000 streams in 168 against
-// 103.  Up to 4,096 q8 rows the passes are one, and 512 x 1,200 x 256 takes 52
-// against 63.
-inline bool stream_is_faster(bool q8, int64_t n, int64_t d, int64_t nq) {
-    const double limit = q8 && n <= 4096 ? 3e8 : 5e8;
-    return (double)nq * (double)n * (double)(d + 256) < limit;
+// rows once per query.  The work of a row and query is its d values and a part
+// (256 of them) that no width saves.  Whole reference calls, cosine, k = 10, us
+// in passes / streaming, by nq x n x d:
+//
+//   the line                32 x 39,877 x 128 q8    56 / 36   8 x 79,753 x 512 q4      65 / 54
+//   past it                 32 x 39,063 x 384 q8    57 / 58   32 x 32,553 x 512 q4     62 / 71
+//   one pass, q8            128 x 3,051 x 512       40 / 40   200 x 2,400 x 384 (3.1e8) 44 / 45
+//   one pass, wide          128 x 1,145 x 768 q8    36 / 38   128 x 2,289 x 768 q4     44 / 53
+//   q8, general kernel      32 x 9,765 x 480        54 / 47   32 x 13,587 x 480        54 / 56
+//                           32 x 5,477 x 600        57 / 50   32 x 8,397 x 600         58 / 66
+//   one pass, the same      32 x 2,921 x 600        40 / 42   128 x 933 x 1,000        49 / 56
+//
+// Up to 4,096 rows the passes are one and cost two thirds of three (q4's a
+// little more than q8's), so less work pays for them, least for wide rows.
+// coalesced: q4, or the q8 kernel of fixed widths; the q8 kernel of any width
+// takes up to twice as long on wide rows.  Where the sides differ little the
+// line is not fitted: 8 x 59,815 x 768 q8 still streams, 66 / 75.
+inline bool stream_is_faster(bool q8, bool coalesced, int64_t n, int64_t d, int64_t nq) {
+    const bool one_pass = n <= 4096;
+    double line = q8 && one_pass ? 3e8 : 5e8;
+    if (one_pass && d > 512) line /= 2;
+    if (!coalesced && d > 256) line /= 2;
+    return (double)nq * (double)n * (double)(d + 256) < line;
 }
 
 }  // namespace manta

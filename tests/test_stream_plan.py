@@ -11,6 +11,9 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 DRIVER = r"""
 #include "stream_plan.hpp"
 extern "C" int rounds(int64_t tiles, int64_t nq, int64_t wgs) { return manta::choose_rounds(tiles, nq, wgs); }
+extern "C" int stream(int q8, int coalesced, int64_t n, int64_t d, int64_t nq) {
+    return manta::stream_is_faster(q8 != 0, coalesced != 0, n, d, nq);
+}
 """
 
 
@@ -23,6 +26,7 @@ def lib(tmp_path_factory):
                     str(so)], check=True)
     lib = C.CDLL(str(so))
     lib.rounds.argtypes = [C.c_int64, C.c_int64, C.c_int64]
+    lib.stream.argtypes = [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64]
     return lib
 
 
@@ -34,3 +38,24 @@ def test_rounds_stay_within_the_rows(lib):
                 assert 1 <= r <= 64 and r <= tiles, (tiles, nq, wgs, r)
                 # as many as spread the work over wgs workgroups, where there are that many
                 assert r >= min(64, tiles, -(-tiles * nq // wgs)), (tiles, nq, wgs, r)
+
+
+# Whole calls timed both ways, us: format, coalesced, n, d, nq, in passes, streaming.
+TIMED = [
+    ("q8", True, 159505, 128, 8, 57, 41), ("q8", True, 23925, 384, 32, 55, 45), ("q8", True, 79753, 512, 8, 59, 50),
+    ("q8", True, 130209, 384, 32, 62, 98), ("q8", True, 79617, 1024, 8, 75, 128), ("q8", True, 11963, 1024, 32, 62, 54),
+    ("q8", True, 500, 256, 512, 39, 29), ("q8", True, 3739, 768, 128, 45, 61), ("q8", True, 1200, 768, 200, 40, 52),
+    ("q8", True, 1200, 1024, 200, 42, 61), ("q8", True, 2400, 768, 200, 44, 73), ("q8", True, 4001, 256, 64, 41, 31),
+    ("q8", False, 28089, 100, 32, 53, 44), ("q8", False, 7959, 333, 32, 52, 38), ("q8", False, 25997, 333, 32, 55, 66),
+    ("q8", False, 25475, 480, 8, 52, 45), ("q8", False, 20805, 480, 32, 57, 74), ("q8", False, 17889, 600, 32, 58, 97),
+    ("q8", False, 12191, 1000, 32, 62, 81), ("q8", False, 2099, 600, 128, 39, 65), ("q8", False, 1867, 1000, 128, 41, 63),
+    ("q8", False, 5477, 600, 32, 57, 50), ("q8", False, 16219, 900, 8, 55, 47), ("q8", False, 3047, 1000, 128, 45, 81),
+    ("q4", True, 39877, 128, 32, 57, 50), ("q4", True, 83221, 480, 8, 64, 59), ("q4", True, 49079, 992, 8, 79, 61),
+    ("q4", True, 39063, 384, 32, 62, 78), ("q4", True, 24415, 768, 32, 68, 90), ("q4", True, 3739, 768, 128, 48, 69),
+    ("q4", True, 2400, 256, 300, 74, 43), ("q4", True, 1200, 768, 300, 53, 67), ("q4", True, 1200, 1024, 300, 72, 111),
+]
+
+
+@pytest.mark.parametrize("fmt,coalesced,n,d,nq,passes,stream", TIMED)
+def test_the_streaming_line_follows_the_times(lib, fmt, coalesced, n, d, nq, passes, stream):
+    assert bool(lib.stream(fmt == "q8", coalesced, n, d, nq)) == (stream < passes)
