@@ -144,3 +144,70 @@ def test_encoder_output_feeds_score_topk(rt):
     want = orc.topk(ref, 25)
     np.testing.assert_array_equal(ids.download(), want)
     np.testing.assert_array_equal(scores.download(), np.take_along_axis(ref, want, 1))
+
+
+def _exact_layers(layers, tokens, mask, tcodes, tscales, packed, r=lambda x: x):
+    """The forward in 64 bits; r: what the operands of the weight products and
+    the output are rounded by."""
+    y = tcodes[tokens].astype(np.float64) * tscales[tokens].astype(np.float64)[..., None]
+    w = [c.astype(np.float64) * s.astype(np.float64)[None, :] for c, s in packed]
+
+    def layernorm(x):
+        x = x - x.mean(-1, keepdims=True)
+        return x / np.sqrt((x * x).mean(-1, keepdims=True) + 1e-5)
+
+    for _ in range(layers):
+        q, k, v = (r(y) @ w[i] for i in range(3))
+        s = q @ k.transpose(0, 2, 1)
+        p = np.exp(s - s.max(-1, keepdims=True))
+        hid = layernorm(r((p / p.sum(-1, keepdims=True)) @ v) @ w[3] + y)
+        up = r(hid) @ w[4]
+        up = 0.5 * up * (1.0 + np.tanh(0.7978845608 * (up + 0.044715 * up ** 3)))
+        y = layernorm(r(up) @ w[5] + hid)
+    y /= np.linalg.norm(y, axis=-1, keepdims=True)
+    m = mask[..., None].astype(np.float64)
+    return r((y * m).sum(1) / np.maximum(m.sum(1), 1.0))
+
+
+@pytest.mark.parametrize("layers", [1, 2])
+@pytest.mark.parametrize("b,t,d,h", [(9, 33, 384, 1536), (40, 64, 256, 512), (3, 200, 128, 512), (512, 64, 384, 256),
+                                     (7, 40, 512, 256)])
+def test_encoder_repeats_and_stays_near_64_bits(rt, b, t, d, h, layers):
+    """The same call gives the same bits among calls on other inputs, and its
+    error against 64 bits stays that of its roundings to f16 (the products'
+    left operands and the output): at most 1.5 times what the same roundings
+    leave of a forward that is otherwise in 64 bits.  The f32 steps round 2^13
+    times finer; what they add is to move a few of those roundings."""
+    case, other = _case(b + t, b, t, 500, d, h), _case(b + t + 1, b, t, 500, d, h)
+    got = [_run_layers(rt, layers, *c).download() for c in (case, other, case, case, other, case)]
+    for i in (2, 3, 5):
+        np.testing.assert_array_equal(got[i], got[0])
+    np.testing.assert_array_equal(got[4], got[1])
+    want = _exact_layers(layers, *case)
+    rounded = _exact_layers(layers, *case, r=lambda x: x.astype(np.float16).astype(np.float64))
+    off = np.linalg.norm(got[0].view(np.float16).astype(np.float64) - want)
+    assert off <= 1.5 * np.linalg.norm(rounded - want), off / np.linalg.norm(want)
+
+
+class _At:
+    """A device array's memory at an odd address."""
+
+    def __init__(self, array, shape, dtype, offset):
+        self.array, self.shape, self.dtype = array, shape, dtype
+        self.addr = array.addr + offset
+
+
+@pytest.mark.parametrize("layers", [1, 2])
+@pytest.mark.parametrize("d,h,t", [(384, 256, 33), (128, 128, 64), (512, 128, 20), (96, 64, 20)])
+def test_encoder_unaligned_table(rt, d, h, t, layers):
+    """Token rows that do not begin on 16 bytes: the same bits (the fused
+    gather and residual take aligned rows only)."""
+    tokens, mask, tcodes, tscales, packed = _case(d + t, 5, t, 60, d, h)
+    want = _run_layers(rt, layers, tokens, mask, tcodes, tscales, packed).download()
+    dev = [(rt.to_device(c), rt.to_device(s)) for c, s in packed]
+    tok, msk, sc = rt.to_device(tokens), rt.to_device(mask), rt.to_device(tscales)
+    for offset in (1, 8):
+        padded = np.concatenate([np.zeros(offset, np.int8), tcodes.reshape(-1)])
+        table = _At(rt.to_device(padded), tcodes.shape, tcodes.dtype, offset)
+        got = rt.encoder_pooled(tok, msk, table, sc, dev, layers=layers).download()
+        np.testing.assert_array_equal(got, want)

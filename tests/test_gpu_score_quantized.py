@@ -93,8 +93,9 @@ def _check_q8_topk(rt, op, smallest, q, codes, scales, k):
 @pytest.mark.parametrize("d", [64, 128, 192, 384, 512, 768, 1024])
 @pytest.mark.parametrize("k", [1, 33, 64])
 def test_q8_wave_list_topk_bit_exact(rt, op, smallest, d, k):
-    """k <= 64 keeps sorted per-wave lists in registers: every coalesced row
-    width, with a row count that leaves a partial last round."""
+    """Sorted per-wave lists in registers (k = 1) and the buffered selection
+    (33, 64): every coalesced row width, with a row count that leaves a partial
+    last round."""
     nq, n = 2, 5000 + d
     q, codes, scales = _q8_case(d + k, nq, n, d, nq)
     _check_q8_topk(rt, op, smallest, q, codes, scales, k)
@@ -102,8 +103,9 @@ def test_q8_wave_list_topk_bit_exact(rt, op, smallest, d, k):
 
 @pytest.mark.parametrize("k", [10, 64])
 def test_q8_wave_list_many_parts(rt, k):
-    """One query over 300000 rows: over a thousand workgroups publish their
-    lists, and the final merge walks all of them."""
+    """One query over 300000 rows: 235 workgroups publish their best keys, and
+    the last merges them all (k = 10 from the lists, 64 from the buffer;
+    tests/test_gpu_wave_lists.py has lists of more than 16)."""
     q, codes, scales = _q8_case(7 + k, 1, 300000, 128, 1)
     _check_q8_topk(rt, "dot", False, q, codes, scales, k)
 
@@ -201,7 +203,9 @@ def test_config0_full_size_bit_exact(rt):
 
 
 # ---------------------------------------------------------------------------
-# Many queries against one shared candidate matrix (the matrix-core path).
+# Many queries against one shared candidate matrix (the matrix-core path;
+# top-k of little work and k <= 192 streams instead, so the smaller shapes here
+# hold both routes to the oracle, and tests/test_gpu_multi_query.py the passes).
 
 @pytest.mark.parametrize("op,smallest", [("dot", False), ("cosine", False), ("l2_distance", True),
                                          ("dot", True), ("l2_distance", False)])
@@ -238,7 +242,8 @@ def test_multi_query_topk_bit_exact(rt, op, smallest, nq, n, d, k):
 def test_multi_query_zero_rows_partial_group(rt, op, smallest):
     """All-zero rows (cosine's zero denominator) among normal ones, with a
     query count that leaves most of the last query group empty: the empty
-    slots never append keys, and zero rows score like the oracle's."""
+    slots never append keys, and zero rows score like the oracle's.  (6,000
+    rows stream; tests/test_gpu_multi_query.py has the passes.)"""
     nq, n, d, k = 19, 6000, 128, 40
     q, codes, scales = _q8_case(91, nq, n, d, sets=1, normalize=(op != "l2_distance"))
     codes, scales = codes[0].copy(), scales[0].copy()
@@ -390,7 +395,8 @@ def test_q8_dot_512_queries_negative_scales(rt):
 
 
 # ---------------------------------------------------------------------------
-# Many queries against one shared q4 matrix (the q4 matrix-core path).
+# Many queries against one shared q4 matrix (the q4 matrix-core path; little
+# work streams, as above).
 
 def _q4_case(seed, nq, n, d, normalize=True):
     q = synth.normal_f16(200 + seed, 0, nq, d, 1.0, normalize=normalize)

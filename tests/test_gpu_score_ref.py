@@ -5,8 +5,8 @@ dequantized candidates, and topKTensor's ids (value desc, index asc).
 Bar: ids and scores bit-exact with the oracle's restatement of those
 functions (oracle.ref_score_q8 / ref_score_q4, pinned against the dequantized
 matrix form in tests/test_oracle_properties.py) on identical seeded inputs,
-through every device route: the streaming scans (per-wave lists and the
-reservoir), the multi-query matrix-core passes, the q4 int8 shadow, the
+through every device route: the streaming scans (per-wave lists, buffered
+selection and the reservoir), the multi-query matrix-core passes, the q4 int8 shadow, the
 reference finish and its full rescan (ties, duplicates, zero rows and
 queries, scales outside the scans' range).
 """
@@ -101,7 +101,8 @@ def test_q4_score_matrix_reference(rt, op, d):
                                    (20000, 100, 256), (5000, 1000, 100)])
 def test_q8_topk_reference_streaming(rt, op, smallest, sets, n, k, d):
     """One query per workgroup (few queries, or one candidate set per query):
-    per-wave lists (k <= 48) and the reservoir, then the finish."""
+    per-wave lists (k <= 16), the buffered selection (up to 192) and the
+    reservoir, then the finish."""
     nq = 4
     q, codes, scales = _q8_case(n + k + d, nq, n, d, sets, normalize=(op != "l2_distance"))
     cands = rt.bind_q8(codes, scales)
@@ -114,8 +115,9 @@ def test_q8_topk_reference_streaming(rt, op, smallest, sets, n, k, d):
 @pytest.mark.parametrize("nq,n,d,k", [(8, 5000, 128, 10), (33, 20000, 384, 50), (16, 30000, 128, 1000),
                                       (40, 4097, 256, 100), (64, 12345, 64, 1), (300, 4000, 256, 20)])
 def test_q8_topk_reference_multi_query(rt, op, smallest, nq, n, d, k):
-    """Many queries against one shared matrix: the matrix-core passes rank
-    the rows, the finish rescores and proves."""
+    """Many queries against one shared matrix: the finish rescores and proves
+    what the scans rank.  k = 1000 takes the matrix-core passes, the small
+    shapes stream (tests/test_gpu_multi_query.py has them past that line)."""
     q, codes, scales = _q8_case(nq + n + d + k, nq, n, d, 1, normalize=(op != "l2_distance"))
     cands = rt.bind_q8(codes, scales)
     _check_topk(rt, cands, op, q, orc.ref_score_q8(op, q, codes, scales), k, smallest)
