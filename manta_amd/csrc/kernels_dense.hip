@@ -7,8 +7,9 @@
 // The order of operations is fixed, so the work cannot be reassociated onto
 // the matrix cores: each (query, row) pair is one sequential chain of
 // v_mul_f32 + v_add_f32, and what bounds many queries is those two
-// instructions per element and pair (64 f32 queries against 200,000 x 384
-// rows: 250 us at the VALU rate, against 63 us to copy the rows).
+// instructions per element and pair: 9.8 G lane instructions for 64 f32 queries
+// against 200,000 x 384 rows, 170 us at the 58 T/s that a loop of nothing but
+// such pairs reaches on this card (63 us to copy the rows).
 //
 // Tiles: a workgroup takes RT rows x QT queries, KC elements of each at a
 // time staged through LDS transposed ([element][row], [element][query]); a
@@ -18,7 +19,9 @@
 // past the common length are staged as zeros on both sides: a partial sum is
 // never -0 (it starts at +0), so adding 0 * 0 leaves it as it is.  A lane
 // reading its own row's 16 bytes at a time (1536 bytes apart), every row again
-// for each 8 queries, took 2,506 us on that shape; these tiles 250-260 us.
+// for each 8 queries, took 2,506 us on that shape; these tiles 242-255 us
+// (the LDS reads, TR + TQ values for 2*TR*TQ instructions, and the staging
+// issue beside them).
 // Output: the f32 score matrix [nq][n] (the top-k runs on it afterwards).
 #include <hip/hip_runtime.h>
 

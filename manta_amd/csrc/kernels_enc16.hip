@@ -130,7 +130,8 @@ hipError_t launch_enc_prep(EncPrepArgs& a, hipStream_t s) {
 }
 
 // x16[i][c] = f16(codes[tok[i]][c] * scale[tok[i]]), 8 columns a thread; an id
-// out of range is recorded in err (flag | id) and its row is zero.
+// out of range is recorded in err (report_gather_error: the first position and
+// its id) and its row is zero.
 __global__ __launch_bounds__(256) void enc_gather16_kernel(const int32_t* __restrict__ tok, int64_t rows,
                                                            const int8_t* __restrict__ codes,
                                                            const float* __restrict__ scales, int64_t vocab, int d,
@@ -184,7 +185,11 @@ hipError_t launch_enc_gather16(const int32_t* tok, int64_t rows, const int8_t* c
 // registers, a row's sums go over its lanes by halving exchanges and over the
 // column groups through LDS (f32 sums of the values, then of the squared
 // deviations; f64 for the row norm), so the product, its sum with the
-// residual and the normalized rows never travel through HBM.
+// residual and the normalized rows never travel through HBM.  What it costs:
+// a wave of the 256 x 384 tile holds 192 accumulators, and the row sums beside
+// them spill (the compiler's report, bytes a lane and registers: layernorm 300
+// and 76, with the token rows as residual 104 and 25, with norm and sums 312 and
+// 82; the other tiles none).
 template <int MT, int NT>
 struct EncTile {
     static constexpr int RG = MT == 256 ? 4 : 2, CG = 8 / RG;

@@ -9,8 +9,10 @@
 // multiplies); a DPP group sum over the L lanes leaves every lane of a group
 // the row total, and lane g*L + j keeps row g*L + j, so after a round each
 // lane owns one row for the epilogue.  The epilogue computes the f32 score
-// and either stores it (score matrix) or offers its key to per-wave sorted
-// register lists (k <= 64) or the LDS reservoir.  In top-k mode each
+// and either stores it (score matrix), offers its key to per-wave sorted
+// register lists (k <= 16, and up to 64 with too many parts for the next),
+// keeps it in LDS for a selection at the end (k <= kBestMaxK), or offers its
+// key to the LDS reservoir.  In top-k mode each
 // workgroup publishes its k best keys; the last workgroup of a query (atomic
 // ticket) merges them into the final ids.
 //
@@ -261,8 +263,8 @@ __device__ __forceinline__ void emit_round(const ScanArgs& a, float score, bool 
     }
 }
 
-// End of a buffered top-k scan workgroup (64 < k <= kBestMaxK): its scores
-// are in LDS, a thread's own rows in its own words, so the rounds ran without
+// End of a buffered top-k scan workgroup (k <= kBestMaxK; on the fixed-width
+// q8 kernel 16 < k, where smaller k takes the wave lists): its scores are in LDS, a thread's own rows in its own words, so the rounds ran without
 // a barrier or an atomic; the k best of them, and of the query's parts, by a
 // floor and ranks.  Against the reservoir (compactions between rounds, the
 // last workgroup streaming every part key through it): one q4 query, 1,048,576

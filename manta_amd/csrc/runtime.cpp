@@ -1659,9 +1659,11 @@ int encoder_f16(MantaRocm* rt, const int32_t* tokens, const int32_t* mask, int64
     // d]; x16 (the gather, then mixed, hid and y rounded) [rows, d]; ffn16
     // [rows, h]; the weights as f16 [N][K], q, k and v one after the other.
     // Without the fused forms also: x [rows, d], the scores [b, t, t].
-    // The column sums of the pooled rows reuse q, k and v ([slabs][slots][d]:
-    // a slab holds at least 32 rows and at most 33 sequences' shares, so even
-    // t = 1 takes less than 3 rows of d per row).
+    // The column sums of the pooled rows reuse q, k and v's space, which is as
+    // large as the larger of the two: 3 rows of d per row, and [slabs][slots][d]
+    // (a slab of 32 or 64 rows holds shares of up to as many sequences; slots is
+    // up to one more, so t = 1 takes one row of d per row and one per slab, and
+    // a single row 33).
     const size_t rd = (size_t)rows * (size_t)d;
     const int slab = manta::enc_pool_slab(rows, d);
     const int slots = (int)((slab - 1) / t) + 2;
