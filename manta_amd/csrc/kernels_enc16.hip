@@ -485,7 +485,9 @@ __global__ __launch_bounds__(512) void enc_gemm16_kernel(EncGemmArgs a) {
     } else {
         // normalizeRows after a layernorm: the layernorm's factor cancels, a
         // row of deviations over its norm (f64 sum of squares as the
-        // reference's norm) is the same row with fewer roundings
+        // reference's norm) is the same row with fewer roundings -- except
+        // where the layernorm's f32 variance overflows: its factor is then 0,
+        // and so is the row (a deviation that is itself infinite: NaN)
 #pragma unroll
         for (int rb = 0; rb < RB; rb++) {
             double ds[16];
@@ -513,7 +515,9 @@ __global__ __launch_bounds__(512) void enc_gemm16_kernel(EncGemmArgs a) {
             double t = dpart[tid];
 #pragma unroll
             for (int c = 1; c < TL::CG; c++) t += dpart[c * MT + tid];
-            rowv[tid] = t > 0.0 ? fminf((float)(1.0 / sqrt(t)), 3.4e38f) : t == 0.0 ? 0.0f : (float)t;
+            if (!(t > 0.0)) rowv[tid] = (float)t;  // 0 or NaN
+            else if ((float)t < __builtin_inff()) rowv[tid] = fminf((float)(1.0 / sqrt(t)), 3.4e38f);
+            else rowv[tid] = t < __builtin_inf() ? 0.0f : __builtin_nanf("");
         }
     }
     __syncthreads();

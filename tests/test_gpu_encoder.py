@@ -211,3 +211,17 @@ def test_encoder_unaligned_table(rt, d, h, t, layers):
         table = _At(rt.to_device(padded), tcodes.shape, tcodes.dtype, offset)
         got = rt.encoder_pooled(tok, msk, table, sc, dev, layers=layers).download()
         np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("layers", [1, 2])
+@pytest.mark.parametrize("b,t,d,h", [(5, 40, 384, 256), (4100, 8, 128, 128), (3, 20, 512, 128), (3, 20, 96, 64)])
+def test_encoder_overflowing_variance(rt, b, t, d, h, layers):
+    """Rows whose layernorm variance overflows in f32 are zero after it, and
+    stay zero through the normalize and the pool (finite deviations)."""
+    tokens, mask, tcodes, tscales, packed = _case(b + t + d, b, t, 50, d, h)
+    packed[5] = (packed[5][0], packed[5][1] * np.float32(1e22))
+    got = _run_layers(rt, layers, tokens, mask, tcodes, tscales, packed).download().view(np.float16)
+    n = min(b, 5)  # (the oracle's time)
+    want = _want_layers(layers, tokens[:n], mask[:n], tcodes, tscales, packed)
+    assert np.all(want == 0.0)
+    assert np.all(got == 0.0)
