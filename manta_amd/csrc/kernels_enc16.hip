@@ -188,8 +188,8 @@ hipError_t launch_enc_gather16(const int32_t* tok, int64_t rows, const int8_t* c
 // residual and the normalized rows never travel through HBM.  What it costs:
 // a wave of the 256 x 384 tile holds 192 accumulators, and the row sums beside
 // them spill (the compiler's report, bytes a lane and registers: layernorm 300
-// and 76, with the token rows as residual 104 and 25, with norm and sums 312 and
-// 82; the other tiles none).
+// and 76, with the token rows as residual 104 and 25, with norm and sums 316 and
+// 84; the other tiles none).
 template <int MT, int NT>
 struct EncTile {
     static constexpr int RG = MT == 256 ? 4 : 2, CG = 8 / RG;

@@ -89,7 +89,8 @@ struct MantaRocmCandidates {
     bool ref_ranked = false;
     mutable size_t bytes = 0;
     bool scales_finite = false;  // every row / block scale is finite (the 512-query kernel needs it)
-    bool scales_nonneg = false;  // q8: no row scale is below zero (the 512-query kernel's pre-filter needs it)
+    bool scales_nonneg = false;  // q8: no row scale is below zero (the 512-query kernel's pre-filter and the
+                                 // cosine passes' need it, and the cosine scans' as a ranking for the reference's)
     // q4: int8 shadow for many-query top-k (built on first use): codes
     // [n][shadow_pitch], scales [2][n] (dot, cosine), error bounds
     mutable int shadow_state = 0;  // 0 not built, 1 built, -1 unavailable
@@ -309,7 +310,7 @@ int free_candidates_memory(MantaRocmCandidates* c) {
 void set_row_maxima(MantaRocmCandidates* c, const std::vector<float>& dnorm, const std::vector<float>& dd) {
     float mn = 0.0f, md = 0.0f;
     for (size_t i = 0; i < dnorm.size(); i++) {
-        mn = std::fmax(mn, dnorm[i]);
+        mn = std::fmax(mn, std::fabs(dnorm[i]));  // (a q8 row of negative scale: negative)
         md = std::fmax(md, dd[i]);
     }
     c->maxdn = mn;
@@ -963,6 +964,9 @@ MqPlan mq_plan(const MantaRocmCandidates* c, int dop, int64_t nq, int64_t k, boo
             mq8_fits(c->pitch, k)) {
             p.sh = manta::mq8_shape(c->pitch, ws8, false);
         } else {
+            // a row of negative scale has a negative |d| in the cosine formula,
+            // which turns the passes' test of q.d against the threshold around
+            if (topk && dop == manta::OP_COSINE && !c->scales_nonneg) return p;
             const int ks = manta::mq_ks(c->pitch);
             if (!ks) return p;
             p.sh = manta::mq_shape(dop, ks, nq);
@@ -1242,14 +1246,16 @@ int scan_topk(MantaRocm* rt, const MantaRocmCandidates* c, int dop, int order, c
 // (or not) that they hold the reference's best k; queries it cannot prove
 // are rescanned in full with the reference arithmetic.  Candidates whose
 // scales lie outside the range the scan's error bounds assume skip the scan
-// and are rescanned in full.
+// and are rescanned in full; so are q8 rows of negative scales for cosine,
+// whose scan scores have the other sign.
 int ref_topk(MantaRocm* rt, const MantaRocmCandidates* c, const ScoreOp& so, int order, const uint16_t* q,
              int64_t nq, int64_t k, int32_t* out_ids, float* out_scores, manta_rt::Scratch* sc, char** err) {
     const int fmt = c->format == MANTA_ROCM_Q8_ROWS ? 8 : 4;
     const int smallest = order == MANTA_ROCM_SMALLEST;
     int* redo = nullptr;
     uint64_t* redo_tau = nullptr;
-    if (c->ref_ranked) {
+    const bool ranked = c->ref_ranked && (fmt == 4 || so.ref != manta::OP_COSINE || c->scales_nonneg);
+    if (ranked) {
         // a margin of rows past the k-th: ties and near-ties of the scan
         // scores across the kp-th row are what would send a query to the
         // full rescan.  A margin that would just pass a power of two stops

@@ -258,3 +258,22 @@ def test_quantized_dot_differs_from_reference_dot(rt):
     np.testing.assert_array_equal(quant, orc.score_q8("dot", q, codes, scales))
     assert not np.array_equal(ref, quant)
     cands.close()
+
+
+@pytest.mark.parametrize("quantized", [False, True])
+@pytest.mark.parametrize("op,smallest", [("dot", False), ("cosine", False), ("cosine", True), ("l2_distance", True)])
+@pytest.mark.parametrize("nq,n,k", [(3, 20000, 30), (40, 45000, 30), (12, 20000, 300)])
+def test_negative_row_scales(rt, nq, n, k, op, smallest, quantized):
+    """Rows of a negative scale, through the streaming scans and the
+    multi-query passes."""
+    d = 128
+    q, codes, scales = _q8_case(37, nq, n, d, 1, normalize=(op != "l2_distance"))
+    scales = scales.copy()
+    scales[np.random.default_rng(37).random(n) < 0.2] *= -1.0
+    cands = rt.bind_q8(codes, scales)
+    want_s = (orc.score_q8 if quantized else orc.ref_score_q8)(op, q, codes, scales)
+    ids, sc, _ = rt.score_topk(cands, op, rt.to_device(q), k, smallest=smallest, quantized=quantized)
+    want = orc.topk(want_s, k, smallest=smallest)
+    np.testing.assert_array_equal(ids.download(), want)
+    np.testing.assert_array_equal(sc.download(), np.take_along_axis(want_s, want, 1))
+    cands.close()
