@@ -2,8 +2,9 @@
 // cosineRows, l2DistanceRows; runtime/backend/tensor_ops.go:1366-1490) on the
 // values packed q8 / q4 rows stand for.
 //
-// ref_rescore_kernel (16 lanes a row): the quantized-query scans return their
-// best kp rows; each is rescored with the reference arithmetic.
+// ref_rescore_kernel (16 lanes a row; ref_rescore_rows_kernel, a row a thread,
+// for many): the quantized-query scans return their best kp rows; each is
+// rescored with the reference arithmetic.
 // ref_finish_kernel (one workgroup per query) sorts them by (score, index)
 // as topKTensor does
 // (tensor_ops.go:1539-1551), and keeps the best k if the bounds of
@@ -289,6 +290,39 @@ __global__ __launch_bounds__(256) void ref_rescore_kernel(RefArgs a, uint64_t* _
         }
     }
     if (has && i16 == 0) keys[(int64_t)q0 * a.kp + at] = ok ? make_key(s, (uint32_t)cid, a.smallest) : 0ull;
+}
+
+// The same with a candidate a thread, grid (ceil(kp / 256), nq): one chain
+// takes d dependent steps however few candidates there are, but every lane
+// works, where above 15 of 16 wait for dot's chain or share a row's sum.
+template <int FMT, int OP>
+__global__ __launch_bounds__(256) void ref_rescore_rows_kernel(RefArgs a, uint64_t* __restrict__ keys) {
+    __shared__ float qf[kMaxQueryDim];
+    __shared__ double sqn_s;
+    const int q = blockIdx.y, d = a.d;
+    const int at = blockIdx.x * 256 + threadIdx.x;
+    const bool has = at < a.kp;
+    const int32_t cid = has ? a.cand_ids[(int64_t)q * a.kp + at] : -1;
+    for (int c = threadIdx.x; c < d; c += 256) qf[c] = h2f(a.queries[(int64_t)q * d + c]);
+    __syncthreads();
+    // cosine: the query's norm, a sequential sum, on the last thread, while the
+    // others sum their rows
+    if (OP == OP_COSINE && threadIdx.x == 255) sqn_s = ref_sqrt_norm(qf, d);
+    const bool ok = cid >= 0 && (int64_t)cid < a.n;
+    const int64_t row = (int64_t)q * a.set_stride + (ok ? cid : 0);
+    const double sqd = OP == OP_COSINE ? a.sqd[row] : 0.0;
+    RefAcc<OP> acc;
+    if (ok) {
+        if (FMT == 8)
+            acc = ref_acc_q8<OP>(qf, (const int8_t*)a.codes + row * a.pitch, ((const float*)a.scales)[row], d);
+        else
+            acc = ref_acc_q4<OP>(qf, (const uint8_t*)a.codes + row * a.pitch,
+                                 (const uint16_t*)a.scales + row * (d / 32), d);
+    }
+    if (OP == OP_COSINE) __syncthreads();
+    if (!has) return;
+    const double sqn = OP == OP_COSINE ? sqn_s : 0.0;
+    keys[(int64_t)q * a.kp + at] = ok ? make_key(acc.finish(sqn, sqd), (uint32_t)cid, a.smallest) : 0ull;
 }
 
 // ------------------------------------------------------- score matrix
@@ -577,8 +611,34 @@ static int next_pow2_host(int x) {
     return p;
 }
 
+// Candidates past which a row a thread is faster (us, 16 lanes a row / a row a
+// thread, by candidates in all):
+//              q8 d 64   384      1,000       q4 d 128  384      1,024
+//   dot    3K  7 / 7    12 / 19  24 / 42      7 / 6   12 / 10   24 / 18
+//         26K  7 / 7    19 / 20  56 / 45     10 / 6   21 / 10   60 / 21
+//        309K 31 / 16  125 / 45 429 / 115    52 / 13 141 / 39  480 / 102
+//   cosine 7K  7 / 7     8 / 21  10 / 48      7 / 7    8 / 11   11 / 23
+//         26K 10 / 9    12 / 24  23 / 54     10 / 8   13 / 15   25 / 31
+//         80K 19 / 9    25 / 23  39 / 48     20 / 9   27 / 16   46 / 32
+//   l2    26K  8 / 8    10 / 22  16 / 48      8 / 7   10 / 12   16 / 23
+//         80K 13 / 9    19 / 24  30 / 49     15 / 9   22 / 16   35 / 30
+//        309K 37 / 17   55 / 49 104 / 114    43 / 17  67 / 43  117 / 111
+// (q8's row a thread reads 16 bytes out of every row per load, so wide rows
+// hold it back; q4 rows are half as long)
+template <int FMT, int OP>
+static int64_t ref_rescore_few(int d) {
+    if (OP == OP_DOT) return FMT == 8 ? 24 * 1024 : 0;
+    if (FMT == 8) return (OP == OP_COSINE ? 200 : 400) * (int64_t)d;
+    return OP == OP_COSINE ? 28 * 1024 : 40 * 1024;
+}
+
 template <int FMT, int OP>
 static hipError_t launch_ref_rescore_op(const RefArgs& a, uint64_t* keys, hipStream_t s) {
+    if ((int64_t)a.nq * a.kp > ref_rescore_few<FMT, OP>(a.d)) {
+        const dim3 grid((unsigned)((a.kp + 255) / 256), (unsigned)a.nq);
+        hipLaunchKernelGGL((ref_rescore_rows_kernel<FMT, OP>), grid, dim3(256), 0, s, a, keys);
+        return hipGetLastError();
+    }
     const dim3 grid((unsigned)((a.kp + 15) / 16), (unsigned)a.nq);
     const size_t lds = (size_t)(1 + (OP == OP_DOT ? 16 : 4)) * ref_row_pitch(a.d) * sizeof(float);
     hipLaunchKernelGGL((ref_rescore_kernel<FMT, OP>), grid, dim3(256), lds, s, a, keys);

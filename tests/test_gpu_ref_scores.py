@@ -98,3 +98,22 @@ def test_rescored_candidates(rt, op, fmt, d, nq, k):
     np.testing.assert_array_equal(ids.download(), want_ids)
     np.testing.assert_array_equal(sc.download(), np.take_along_axis(want, want_ids, 1))
     cands.close()
+
+
+@pytest.mark.parametrize("fmt,op,d,nq,k", [("q8", "dot", 100, 130, 200), ("q8", "dot", 1024, 90, 300),
+                                           ("q8", "cosine", 40, 90, 100), ("q8", "cosine", 128, 130, 256),
+                                           ("q8", "l2_distance", 24, 100, 150), ("q8", "l2_distance", 100, 140, 300),
+                                           ("q4", "dot", 96, 1, 1), ("q4", "dot", 1024, 9, 260),
+                                           ("q4", "cosine", 160, 140, 220), ("q4", "l2_distance", 64, 190, 230)])
+def test_many_rescored_candidates(rt, fmt, op, d, nq, k):
+    """Past the line where a row a thread rescores them."""
+    n = 1500
+    q = _queries(d + nq, nq, d)
+    cands, codes, scales = _bind(rt, fmt, d + nq, n, d)
+    want = _want(fmt, op, q, codes, scales)
+    smallest = op == "l2_distance"
+    ids, sc, _ = rt.score_topk(cands, op, rt.to_device(q), k, smallest=smallest)
+    want_ids = orc.topk(want, k, smallest=smallest)
+    np.testing.assert_array_equal(ids.download(), want_ids)
+    np.testing.assert_array_equal(sc.download(), np.take_along_axis(want, want_ids, 1))
+    cands.close()
