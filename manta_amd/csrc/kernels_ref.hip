@@ -694,8 +694,12 @@ template <int FMT, int OP>
 static hipError_t launch_ref_scores_op(const RefArgs& a, float* out, hipStream_t s) {
     const int nq = a.set_stride ? 1 : a.nq;
     const bool few = a.n * nq < 512 * 1024;
-    if (nq > 8 && !few) return launch_ref_scores_tile<FMT, OP, 4, 4, 64>(a, out, s);
+    // (16 queries of rows past 736 columns hold over 64 KB of LDS, one workgroup
+    // a CU: two tiles of 8 instead)
+    if (nq > 8 && !few && a.d <= 736) return launch_ref_scores_tile<FMT, OP, 4, 4, 64>(a, out, s);
     if (nq > 4 && !few) return launch_ref_scores_tile<FMT, OP, 4, 2, 64>(a, out, s);
+    // (stages of 128 columns would be half empty at the end of these rows)
+    if (nq > 4 && ((a.d + 63) / 64) % 2 != 0) return launch_ref_scores_tile<FMT, OP, 8, 1, 64>(a, out, s);
     if (nq > 4) return launch_ref_scores_tile<FMT, OP, 8, 1, 128>(a, out, s);
     const int64_t rows = a.set_stride ? a.n * a.nq : a.n;
     if (nq > 1 || rows < 64 * 1024) return launch_ref_scores_tile<FMT, OP, 4, 1, 64>(a, out, s);

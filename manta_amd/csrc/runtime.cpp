@@ -1152,7 +1152,15 @@ int manta_rocm_score(MantaRocm* rt, const MantaRocmCandidates* c, int op, const 
         // otherwise, and for few rows, tiles of rows and queries through LDS
         // (one x 60,000, d 384: 9.3 and 11; four x 5,000: 36.9 and 12.4)
         const int fmt = c->format == MANTA_ROCM_Q8_ROWS ? 8 : 4;
-        if (fmt == 4 && (nq <= 2 || c->sets > 1) && c->n * nq >= 32768) {
+        // (dot and the l2 of longer rows also for up to 65,536 scores in all: 64
+        // queries x 300, dot, d 128 4.4 and 5.0, 8 x 4,000, l2, d 1024 20.9 and
+        // 23.1; 4 x 20,000, dot, d 128 5.0 and 4.9).  One query over many wide q8
+        // rows, dot and l2, likewise (300,000 x 384: 44.5 and 46.6, x 1,024: 105
+        // and 114).
+        bool lanes = fmt == 4 && (nq <= 2 || c->sets > 1) && c->n * nq >= 32768;
+        if (fmt == 4 && c->n * nq <= 65536) lanes |= so.ref == manta::OP_DOT || (so.ref == manta::OP_L2 && c->d > 128);
+        if (fmt == 8 && nq == 1 && c->n >= 262144 && c->d > 256) lanes = so.ref != manta::OP_COSINE;
+        if (lanes) {
             ScanArgs a = scan_args(c, q);
             a.rounds = (int)std::max<int64_t>(1, std::min<int64_t>(16, tiles * nq / 2048));
             a.out_scores = out;
