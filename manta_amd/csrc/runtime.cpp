@@ -1219,20 +1219,31 @@ int scan_topk(MantaRocm* rt, const MantaRocmCandidates* c, int dop, int order, c
                        "q8_rescore");
         return MANTA_ROCM_OK;
     }
-    StreamTopk st = stream_topk_shape(c, nq, k, manta::choose_rounds((c->n + 255) / 256, nq, rt->cus));
+    const int64_t tiles = (c->n + 255) / 256;
+    StreamTopk st = stream_topk_shape(c, nq, k, manta::choose_rounds(tiles, nq, rt->cus));
+    // small k on the coalesced q8 kernel: sorted per-wave lists in registers
+    // (LDS keys only for merging the waves' lists).  Else the scores of the
+    // workgroup in LDS (a word per row), selected at the end.  A list's offers
+    // and merges grow with k, and with the parts once their keys are more than
+    // the threads (us, lists / buffered):
+    //   one x 65,536 x 256   k = 10 12.9 / 14.7   k = 50 36.9 / 16.4
+    //   32 x 65,536 x 256    k = 10 79.2 / 87.4   k = 50 93.5 / 89.4
+    //   64 x 20,000 x 128, 4 parts    k = 24 31.7 / 35.1   k = 48 37.8 / 35.6
+    //   20 x 6,000 x 384, 12 parts    k = 18 18.4 / 19.6   k = 24 21.4 / 20.1
+    //   64 x 2,500 x 384, 4 parts     k = 32 20.5 / 21.3   k = 48 23.5 / 22.2
+    //   one x 20,000 x 128, 40 parts  k = 12 10.2 / -      k = 18 15.2 / 12.7
+    //   4 x 300 x 384, two tiles      k = 18 10.7 / 14.4   k = 48 13.0 / 15.0
+    const bool lists_fit = c->format == MANTA_ROCM_Q8_ROWS && manta::q8_scan_coalesced(c->pitch) &&
+                           k <= manta::kWaveListMaxK;
+    const bool lists_better = k <= 16 || (k <= (c->pitch >= 384 ? 32 : 24) && st.parts * k <= 256) ||
+                              (k <= 48 && tiles <= 2);
+    const bool buffer_fits = k <= manta::kBestMaxK && st.parts <= manta::kBestMaxParts;
+    const bool lists = lists_fit && (lists_better || !buffer_fits);
     uint64_t* partial = nullptr;
     int rc = take_buffer(rt, sc, (size_t)nq * st.parts * k * 8, (void**)&partial, err);
     if (rc) return rc;
     ScanArgs a = stream_topk_args(c, q, st, k, order, out_ids, out_scores, partial, sc ? sc->tickets : rt->tickets);
-    // k <= 16 on the coalesced q8 kernel: sorted per-wave lists in registers
-    // (LDS keys only for merging the waves' lists).  Larger k: the scores of
-    // the workgroup in LDS (a word per row), selected at the end.  32 problems
-    // of 65,536 x 256: 79.2 (lists) against 87.4 us (buffered) for k = 10, 93.5
-    // against 89.4 for k = 50; one of them 12.9 against 14.7, 36.9 against 16.4.
-    const bool lists_fit = c->format == MANTA_ROCM_Q8_ROWS && manta::q8_scan_coalesced(c->pitch) &&
-                           k <= manta::kWaveListMaxK;
-    const bool buffer_fits = k <= manta::kBestMaxK && st.parts <= manta::kBestMaxParts;
-    if (lists_fit && (k <= 16 || !buffer_fits)) {
+    if (lists) {
         a.wave_lists = 1;
         a.lds_keys = 256;
     } else if (buffer_fits) {

@@ -81,3 +81,18 @@ def test_buffered_selection(rt, fmt, rows, n, k):
         want = orc.score_q8("dot", q, codes, f.astype(np.float32))
     _check(rt, cands, want, "dot", q, min(k, n))
     cands.close()
+
+
+@pytest.mark.parametrize("sets,n,k", [(3, 300, 64), (64, 500, 20), (20, 6000, 21), (20, 6000, 22), (2, 256, 33)])
+def test_q8_lists_of_few_parts(rt, sets, n, k):
+    """Lists and buffered selections on both sides of the line, a set each."""
+    d = 128
+    codes = np.empty((sets, n, d), np.int8)
+    scales = np.empty((sets, n), np.float32)
+    for s in range(sets):
+        codes[s], scales[s] = synth.q8_rows(55, 1 + s, n, d)
+    codes[:, n // 2:] = codes[:, :n - n // 2]  # ties
+    q = synth.normal_f16(55, 0, sets, d, 1.0)
+    cands = rt.bind_q8(codes, scales)
+    _check(rt, cands, orc.score_q8("dot", q, codes, scales), "dot", q, k)
+    cands.close()
