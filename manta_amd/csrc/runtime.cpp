@@ -1239,6 +1239,9 @@ int scan_topk(MantaRocm* rt, const MantaRocmCandidates* c, int dop, int order, c
                               (k <= 48 && tiles <= 2);
     const bool buffer_fits = k <= manta::kBestMaxK && st.parts <= manta::kBestMaxParts;
     const bool lists = lists_fit && (lists_better || !buffer_fits);
+    if (!lists && buffer_fits)
+        st = stream_topk_shape(c, nq, k,
+                               manta::buffered_rounds(tiles, nq, rt->cus, st.rounds, manta::kBestMaxParts, c->pitch));
     uint64_t* partial = nullptr;
     int rc = take_buffer(rt, sc, (size_t)nq * st.parts * k * 8, (void**)&partial, err);
     if (rc) return rc;

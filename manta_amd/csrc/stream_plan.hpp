@@ -26,6 +26,27 @@ inline int choose_rounds(int64_t tiles, int64_t nq, int64_t wgs) {
     return (int)std::max<int64_t>(1, std::min<int64_t>({64, r, tiles}));
 }
 
+// Rounds of a selection that buffers its scores, `pitch` bytes a row.  A
+// workgroup holds a KB of LDS a round (and up to 80 KB beside them), so at the
+// rounds that spread the rows over one workgroup per CU a CU may take no
+// second one, and the few workgroups past a whole wave cost another: 43 parts
+// for each of 6 queries are 258 on 256 CUs.  Parts that make one or two whole
+// waves, where those are not too long for the row's width; else short parts,
+// many a CU.  Before and now, us, q4 dot, k = 5: 6 x 700,000 x 384 321 and 163,
+// 7 x 700,000 x 384 330 and 146, 7 x 1,200,000 x 384 485 and 322.
+inline int buffered_rounds(int64_t tiles, int64_t nq, int64_t wgs, int rounds, int64_t max_parts, int pitch) {
+    if (nq * ((tiles + rounds - 1) / rounds) <= wgs) return rounds;
+    for (int waves = 1; waves <= 2; waves++) {
+        const int64_t parts = std::min(tiles, wgs * waves / nq);
+        if (parts < 1 || parts > max_parts) continue;
+        const int64_t r = (tiles + parts - 1) / parts;
+        // (narrow rows want more wavefronts in flight than one workgroup's;
+        // wide ones keep the memory busy with it)
+        if (r <= (waves == 1 ? (pitch >= 128 ? 64 : 0) : (pitch >= 320 ? 64 : 40))) return (int)r;
+    }
+    return (int)std::min<int64_t>(rounds, std::max<int64_t>(24, (tiles + max_parts - 1) / max_parts));
+}
+
 // Little work: the multi-query passes' launches (encoding, then a scan and a
 // select each) would cost more than one streaming launch that reads the cached
 // rows once per query.  The work of a row and query is its d values and a part

@@ -11,6 +11,9 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 DRIVER = r"""
 #include "stream_plan.hpp"
 extern "C" int rounds(int64_t tiles, int64_t nq, int64_t wgs) { return manta::choose_rounds(tiles, nq, wgs); }
+extern "C" int buffered(int64_t tiles, int64_t nq, int64_t wgs, int rounds, int pitch) {
+    return manta::buffered_rounds(tiles, nq, wgs, rounds, 512, pitch);
+}
 extern "C" int stream(int q8, int coalesced, int64_t n, int64_t d, int64_t nq) {
     return manta::stream_is_faster(q8 != 0, coalesced != 0, n, d, nq);
 }
@@ -26,6 +29,7 @@ def lib(tmp_path_factory):
                     str(so)], check=True)
     lib = C.CDLL(str(so))
     lib.rounds.argtypes = [C.c_int64, C.c_int64, C.c_int64]
+    lib.buffered.argtypes = [C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int]
     lib.stream.argtypes = [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64]
     return lib
 
@@ -38,6 +42,22 @@ def test_rounds_stay_within_the_rows(lib):
                 assert 1 <= r <= 64 and r <= tiles, (tiles, nq, wgs, r)
                 # as many as spread the work over wgs workgroups, where there are that many
                 assert r >= min(64, tiles, -(-tiles * nq // wgs)), (tiles, nq, wgs, r)
+
+
+def test_buffered_rounds_leave_no_short_wave_of_long_parts(lib):
+    """Few workgroups past a whole wave only where the parts are short."""
+    for tiles in (1, 5, 16, 100, 1013, 1172, 2735, 4688, 9766, 19531, 32768):
+        for nq in (1, 2, 3, 5, 6, 7, 20, 64, 300, 1000):
+            for pitch in (16, 32, 64, 128, 192, 336, 1008):
+                rounds = lib.rounds(tiles, nq, 256)
+                r = lib.buffered(tiles, nq, 256, rounds, pitch)
+                parts, most = -(-tiles // r), max(512, -(-tiles // rounds))
+                assert 1 <= r <= min(64, tiles) and parts <= most, (tiles, nq, pitch, rounds, r)
+                short = max(24, -(-tiles // 512))
+                assert r <= short or nq * parts <= 512, (tiles, nq, pitch, rounds, r)
+                if nq * -(-tiles // rounds) <= 256:
+                    assert r == rounds
+    assert lib.buffered(2735, 6, 256, 64, 32) == 33
 
 
 # Whole calls timed both ways, us: format, coalesced, n, d, nq, in passes, streaming.
