@@ -772,6 +772,48 @@ __global__ __launch_bounds__(256) void q8_scan_generic_kernel(ScanArgs a) {
     else if (!a.out_scores) finish_topk(a, topk_keys, S, qi);
 }
 
+// ------------------------------------------------ q8, any pitch (lane = row)
+
+// A row per lane, 16 bytes of every row per load.  The rows' lines come from
+// the caches after their first load; nothing is traded between lanes
+// (q8_row_per_lane: where it is the faster one).
+template <int OP>
+__global__ __launch_bounds__(256) void q8_scan_rows_kernel(ScanArgs a) {
+    extern __shared__ uint64_t topk_keys[];
+    __shared__ ScanLds S;
+    const int qi = blockIdx.y;
+    const int64_t set_row0 = (int64_t)qi * a.set_stride;
+    const int8_t* __restrict__ codes = a.codes + set_row0 * a.pitch;
+    const float* __restrict__ scales = (const float*)a.scales + set_row0;
+    encode_query_block(a.queries + (int64_t)qi * a.d, a.d, a.pitch, OP == OP_DOT ? ENC_E8 : ENC_E16, S.q);
+    const QConst kq = S.q.qc;
+    const int8_t* qa = OP == OP_DOT ? S.q.c8 : S.q.hi;
+    const int8_t* qb = S.q.lo;
+    const int chunks = a.pitch / 16;
+    if (!a.out_scores && !a.buffered) topk_init(topk_keys, &S.st);
+    const int64_t wg_row0 = (int64_t)blockIdx.x * a.rounds * 256;
+    for (int r = 0; r < a.rounds; r++) {
+        const int64_t row = wg_row0 + (int64_t)r * 256 + threadIdx.x;
+        const bool valid = row < a.n;
+        float score = 0.0f;
+        if (valid) {
+            const v4i* rp = (const v4i*)(codes + row * a.pitch);
+            int s_hi = 0, s_lo = 0;
+            for (int c = 0; c < chunks; c++) {
+                const v4i v = rp[c];
+                s_hi = dot16(v, *(const v4i*)(qa + c * 16), s_hi);
+                if (OP != OP_DOT) s_lo = dot16(v, *(const v4i*)(qb + c * 16), s_lo);
+            }
+            const float dn = OP == OP_COSINE ? a.dnorm[set_row0 + row] : 0.0f;
+            const float d2 = OP == OP_L2 ? a.dd[set_row0 + row] : 0.0f;
+            score = q8_epilogue<OP>(s_hi, s_lo, scales[row], kq, dn, d2);
+        }
+        emit_round(a, score, valid, row, r, qi, topk_keys, &S.st);
+    }
+    if (a.buffered) finish_buffered(a, topk_keys, qi);
+    else if (!a.out_scores) finish_topk(a, topk_keys, S, qi);
+}
+
 // ------------------------------------------------------- q4, lane = block
 
 // Lane p of a group of nb lanes takes block p of a row, so a load instruction
@@ -868,6 +910,37 @@ __global__ __launch_bounds__(256) void q4_scan_kernel(ScanArgs a) {
     else if (!a.out_scores) finish_topk(a, topk_keys, S, qi);
 }
 
+// A row per lane: no pairs go through LDS, each lane runs its row's chain
+// (q4_row_per_lane: where it is the faster one).
+template <int OP>
+__global__ __launch_bounds__(256) void q4_scan_rows_kernel(ScanArgs a) {
+    extern __shared__ uint64_t topk_keys[];
+    __shared__ ScanLds S;
+    const int qi = blockIdx.y;
+    const int64_t set_row0 = (int64_t)qi * a.set_stride;
+    const uint8_t* __restrict__ packed = (const uint8_t*)a.codes + set_row0 * a.pitch;
+    const uint16_t* __restrict__ scales = (const uint16_t*)a.scales + set_row0 * a.nb;
+    encode_query_block(a.queries + (int64_t)qi * a.d, a.d, a.d, ENC_E16_Q4, S.q);
+    const QConst kq = S.q.qc;
+    if (!a.out_scores && !a.buffered) topk_init(topk_keys, &S.st);
+    const int64_t wg_row0 = (int64_t)blockIdx.x * a.rounds * 256;
+    for (int r = 0; r < a.rounds; r++) {
+        const int64_t row = wg_row0 + (int64_t)r * 256 + threadIdx.x;
+        const bool valid = row < a.n;
+        float score = 0.0f;
+        if (valid) {
+            const float dotf = q4_row_dotf(packed + row * a.pitch, scales + row * a.nb, a.nb, (const int*)S.q.hi,
+                                           (const int*)S.q.lo);
+            const float dn = OP == OP_COSINE ? a.dnorm[set_row0 + row] : 0.0f;
+            const float d2 = OP == OP_L2 ? a.dd[set_row0 + row] : 0.0f;
+            score = q4_finish<OP>(dotf, kq, dn, d2);
+        }
+        emit_round(a, score, valid, row, r, qi, topk_keys, &S.st);
+    }
+    if (a.buffered) finish_buffered(a, topk_keys, qi);
+    else if (!a.out_scores) finish_topk(a, topk_keys, S, qi);
+}
+
 // ------------------------------------------------ exact accumulator rescore
 
 // One workgroup per query: re-encode the query and recompute the q8
@@ -916,6 +989,42 @@ bool q8_scan_coalesced(int pitch) {
                                chunks == 32 || chunks == 48 || chunks == 64);
 }
 
+// A row per lane, or the pieces of a row side by side over the lanes.  A row
+// per lane reads 16 bytes out of every row at a time: fine while the rows stay
+// in the caches between its loads, and it trades no sums between lanes.  Whole
+// calls, us, row per lane / pieces, dot, k = 8, queries x rows:
+//   q8, d           1 x 30,000    7 x 150,000   1 x 500,000   7 x 500,000   3 x 1,500,000
+//    40 (48 bytes)  11.0 / 13.3   27.1 / 35.4   16.3 / 23.4   44.7 / 54.4   47.7 / 62.6
+//   100             11.8 / 13.5   35.5 / 35.9   23.2 / 23.7  105.8 / 77.7  126.1 / 66.6
+//   200             12.8 / 14.7   47.0 / 49.5   29.6 / 29.4  111.6 / 116.7 158.1 / 111.7
+//   400             14.2 / 18.8   76.6 / 81.8   44.1 / 44.5  160.8 / 221.1
+//   600             16.1 / 25.4  114.7 / 145.3  79.0 / 72.1  311.4 / 403.9
+//   1,000           21.6 / 28.6  177.5 / 176.4  (7 x 300,000, k = 5: 372 / 284)
+//   q4, d
+//    64             11.2 / 13.2   21.5 / 32.7   16.1 / 22.1   33.1 / 50.2   36.0 / 57.0
+//   160             12.0 / 13.9   30.0 / 36.6   20.8 / 24.0   60.7 / 67.7   64.5 / 75.4
+//   256             13.1 / 14.2   40.7 / 40.1   25.9 / 25.8   99.2 / 90.8  104.8 / 95.7
+//   384             13.9 / 16.2   57.8 / 63.5   34.7 / 36.2  142.9 / 156.0 177.6 / 158.0
+//   512             16.4 / 17.4   72.7 / 63.5   41.5 / 39.4  193.9 / 160.6 258.9 / 217.7
+//   1,024           22.0 / 23.6  135.1 / 113.6  84.5 / 64.0  434.9 / 295.6
+constexpr int64_t kMB = 1 << 20;
+
+static bool q8_row_per_lane(const ScanArgs& a, int64_t nq) {
+    const int chunks = a.pitch / 16;
+    if (chunks <= 3) return true;
+    const int64_t one = a.n * a.pitch, all = one * nq, rows = a.set_stride ? all : one;  // bytes: read, and distinct
+    // (33 to 52 pieces: a load takes one row and leaves up to half the lanes idle)
+    if (chunks > 32 && chunks <= 52 && nq > 1 && !a.set_stride) return true;
+    return rows < (chunks > 52 ? 160 : 256) * kMB && (chunks > 8 || all < 80 * kMB);
+}
+
+static bool q4_row_per_lane(const ScanArgs& a, int64_t nq) {
+    if (a.nb <= 5) return true;
+    const int64_t one = a.n * a.pitch, all = one * nq, rows = a.set_stride ? all : one;
+    // (8 blocks: every row starts on the same few cache sets, as 16 and 32 do)
+    return a.nb <= 12 && a.nb != 8 ? rows < 128 * kMB : all < 32 * kMB;
+}
+
 template <int OP>
 static hipError_t launch_q8_op(const ScanArgs& a, dim3 grid, size_t lds, hipStream_t s) {
     const int chunks = a.pitch / 16;
@@ -941,6 +1050,10 @@ static hipError_t launch_q8_op(const ScanArgs& a, dim3 grid, size_t lds, hipStre
     MANTA_Q8(16, 4)   // 1024
 #undef MANTA_Q8
     if (chunks < 1 || chunks > 64 || a.pitch != 16 * chunks || lds < (size_t)a.lds_keys * 8) return hipErrorInvalidValue;
+    if (q8_row_per_lane(a, grid.y)) {
+        hipLaunchKernelGGL((q8_scan_rows_kernel<OP>), grid, dim3(256), lds, s, a);
+        return hipGetLastError();
+    }
     const size_t all = (size_t)a.lds_keys * 8 + (size_t)4 * q8_generic_words(chunks) * sizeof(int2);
     hipLaunchKernelGGL((q8_scan_generic_kernel<OP>), grid, dim3(256), all, s, a);
     return hipGetLastError();
@@ -955,15 +1068,24 @@ hipError_t launch_q8_scan(int op, const ScanArgs& a, dim3 grid, size_t lds, hipS
     }
 }
 
+template <int OP>
+static hipError_t launch_q4_op(const ScanArgs& a, dim3 grid, size_t lds, hipStream_t s) {
+    if (q4_row_per_lane(a, grid.y)) {
+        hipLaunchKernelGGL((q4_scan_rows_kernel<OP>), grid, dim3(256), lds, s, a);
+        return hipGetLastError();
+    }
+    const size_t all = (size_t)a.lds_keys * 8 + (size_t)4 * 64 * (a.nb | 1) * sizeof(float2);  // + (scale, sum) pairs
+    hipLaunchKernelGGL((q4_scan_kernel<OP>), grid, dim3(256), all, s, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_q4_scan(int op, const ScanArgs& a, dim3 grid, size_t lds, hipStream_t s) {
     if (a.nb < 1 || a.nb > 32 || a.pitch != 16 * a.nb || lds < (size_t)a.lds_keys * 8) return hipErrorInvalidValue;
-    const size_t all = (size_t)a.lds_keys * 8 + (size_t)4 * 64 * (a.nb | 1) * sizeof(float2);  // + (scale, sum) pairs
     switch (op) {
-        case OP_DOT: hipLaunchKernelGGL((q4_scan_kernel<OP_DOT>), grid, dim3(256), all, s, a); break;
-        case OP_COSINE: hipLaunchKernelGGL((q4_scan_kernel<OP_COSINE>), grid, dim3(256), all, s, a); break;
-        default: hipLaunchKernelGGL((q4_scan_kernel<OP_L2>), grid, dim3(256), all, s, a); break;
+        case OP_DOT: return launch_q4_op<OP_DOT>(a, grid, lds, s);
+        case OP_COSINE: return launch_q4_op<OP_COSINE>(a, grid, lds, s);
+        default: return launch_q4_op<OP_L2>(a, grid, lds, s);
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_q8_rescore(const int8_t* codes, int pitch, int64_t set_stride, int64_t n, int d,

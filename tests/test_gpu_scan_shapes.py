@@ -83,6 +83,35 @@ def test_buffered_selection(rt, fmt, rows, n, k):
     cands.close()
 
 
+def _tiled_rows(rows, n):
+    """n rows that repeat `rows` with scales of their own, so that the oracle
+    scores few rows and the device reads many."""
+    return np.tile(rows, (-(-n // len(rows)), 1))[:n]
+
+
+@pytest.mark.parametrize("op,k", [("dot", 12), ("cosine", 100), ("l2_distance", 250)])
+@pytest.mark.parametrize("fmt,d,nq,n", [("q8", 100, 4, 500001), ("q8", 500, 1, 530001), ("q8", 840, 1, 330001),
+                                        ("q4", 256, 1, 1050001), ("q4", 416, 2, 90001), ("q4", 1024, 3, 22001)])
+def test_rows_in_pieces(rt, fmt, d, nq, n, op, k):
+    """Past the line where a row per lane streams them (the widths above are
+    below it), in pieces of 16 bytes."""
+    rng = np.random.default_rng(d)
+    q = synth.normal_f16(54, d, nq, d, 1.0)
+    if fmt == "q8":
+        codes = _tiled_rows(rng.integers(-127, 128, (20011, d), dtype=np.int8), n)
+        scales = rng.uniform(0.5, 1.5, n).astype(np.float32) / np.float32(127 * 30)
+        cands = rt.bind_q8(codes, scales)
+        want = orc.score_q8(op, q, codes, scales)
+    else:
+        nib = rng.integers(-7, 8, (20011, d), dtype=np.int8).view(np.uint8) & 15
+        packed = _tiled_rows(nib[:, 0::2] | (nib[:, 1::2] << 4), n)
+        scales = (rng.uniform(0.5, 1.5, (n, d // 32)) / 200).astype(np.float16).view(np.uint16)
+        cands = rt.bind_q4(packed, scales, d)
+        want = orc.score_q4(op, q, packed, scales, d)
+    _check(rt, cands, want, op, q, k)
+    cands.close()
+
+
 @pytest.mark.parametrize("sets,n,k", [(3, 300, 64), (64, 500, 20), (20, 6000, 21), (20, 6000, 22), (2, 256, 33)])
 def test_q8_lists_of_few_parts(rt, sets, n, k):
     """Lists and buffered selections on both sides of the line, a set each."""
