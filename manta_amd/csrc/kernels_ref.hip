@@ -695,7 +695,8 @@ static hipError_t launch_ref_scores_op(const RefArgs& a, float* out, hipStream_t
     const int nq = a.set_stride ? 1 : a.nq;
     const bool few = a.n * nq < 512 * 1024;
     // (16 queries of rows past 736 columns hold over 64 KB of LDS, one workgroup
-    // a CU: two tiles of 8 instead)
+    // a CU: two tiles of 8 instead.  10 q4 queries x 118,304 x 1,024, dot: 334 us,
+    // now 175)
     if (nq > 8 && !few && a.d <= 736) return launch_ref_scores_tile<FMT, OP, 4, 4, 64>(a, out, s);
     if (nq > 4 && !few) return launch_ref_scores_tile<FMT, OP, 4, 2, 64>(a, out, s);
     // (stages of 128 columns would be half empty at the end of these rows)
