@@ -10,10 +10,9 @@
 // the row total, and lane g*L + j keeps row g*L + j, so after a round each
 // lane owns one row for the epilogue.  The epilogue computes the f32 score
 // and either stores it (score matrix), offers its key to per-wave sorted
-// register lists (k <= 16, and up to 64 with too many parts for the next),
+// register lists (small k, and up to 64 with too many parts for the next),
 // keeps it in LDS for a selection at the end (k <= kBestMaxK), or offers its
-// key to the LDS reservoir.  In top-k mode each
-// workgroup publishes its k best keys; the last workgroup of a query (atomic
+// key to the LDS reservoir.  In top-k mode each workgroup publishes its k best keys; the last workgroup of a query (atomic
 // ticket) merges them into the final ids.
 //
 // Quantized-query scores (the CPU oracle restates them):
@@ -264,9 +263,10 @@ __device__ __forceinline__ void emit_round(const ScanArgs& a, float score, bool 
 }
 
 // End of a buffered top-k scan workgroup (k <= kBestMaxK; on the fixed-width
-// q8 kernel 16 < k, where smaller k takes the wave lists): its scores are in LDS, a thread's own rows in its own words, so the rounds ran without
-// a barrier or an atomic; the k best of them, and of the query's parts, by a
-// floor and ranks.  Against the reservoir (compactions between rounds, the
+// q8 kernel, k past the wave lists'): its scores are in LDS, a thread's own
+// rows in its own words, so the rounds ran without a barrier or an atomic; the
+// k best of them, and of the query's parts, by a floor and ranks.  Against the
+// reservoir (compactions between rounds, the
 // last workgroup streaming every part key through it): one q4 query, 1,048,576
 // rows, k = 108, 159 -> 65 us.
 __device__ __forceinline__ void finish_buffered(const ScanArgs& a, const uint64_t* buf, int qi) {

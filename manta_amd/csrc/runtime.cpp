@@ -904,9 +904,7 @@ bool mq8_fits(int pitch, int64_t k) {
 // A top-k that streams one query per workgroup although the passes could take
 // it (k past kBestMaxK streams through the reservoir: the passes).
 bool stream_is_faster(const MantaRocmCandidates* c, int64_t nq, int64_t k) {
-    const bool q8 = c->format == MANTA_ROCM_Q8_ROWS;
-    return k <= manta::kBestMaxK &&
-           manta::stream_is_faster(q8, !q8 || manta::q8_scan_coalesced(c->pitch), c->n, c->d, nq);
+    return k <= manta::kBestMaxK && manta::stream_is_faster(c->format == MANTA_ROCM_Q8_ROWS, c->n, c->d, nq);
 }
 
 // q4 cosine / dot top-k with at least 256 queries goes through the int8

@@ -53,24 +53,23 @@ inline int buffered_rounds(int64_t tiles, int64_t nq, int64_t wgs, int rounds, i
 // (256 of them) that no width saves.  Whole reference calls, cosine, k = 10, us
 // in passes / streaming, by nq x n x d:
 //
-//   the line                32 x 39,877 x 128 q8    56 / 36   8 x 79,753 x 512 q4      65 / 54
-//   past it                 32 x 39,063 x 384 q8    57 / 58   32 x 32,553 x 512 q4     62 / 71
-//   one pass, q8            128 x 3,051 x 512       40 / 40   200 x 2,400 x 384 (3.1e8) 44 / 45
-//   one pass, wide          128 x 1,145 x 768 q8    36 / 38   128 x 2,289 x 768 q4     44 / 53
-//   q8, general kernel      32 x 9,765 x 480        54 / 47   32 x 13,587 x 480        54 / 56
-//                           32 x 5,477 x 600        57 / 50   32 x 8,397 x 600         58 / 66
-//   one pass, the same      32 x 2,921 x 600        40 / 42   128 x 933 x 1,000        49 / 56
+//   inside       32 x 39,877 x 128 q8   55 / 36    32 x 17,889 x 600 q8   59 / 55
+//                8 x 79,753 x 512 q4    64 / 54    32 x 12,191 x 1,000 q8 62 / 55
+//   past it      32 x 39,063 x 384 q8   57 / 55    8 x 156,251 x 384 q8   62 / 99
+//                32 x 32,553 x 512 q4   62 / 70    32 x 24,415 x 768 q8   65 / 65
+//   one pass     128 x 3,397 x 480 q8   43 / 44    200 x 2,400 x 384 q8   43 / 47
+//                512 x 1,200 x 256 q8   40 / 33    300 x 2,400 x 256 q4   74 / 42
+//   ... wide     128 x 1,145 x 768 q8   37 / 35    200 x 1,200 x 768 q8   39 / 52
+//                128 x 1,013 x 900 q8   40 / 35    128 x 2,289 x 768 q4   43 / 53
 //
 // Up to 4,096 rows the passes are one and cost two thirds of three (q4's a
 // little more than q8's), so less work pays for them, least for wide rows.
-// coalesced: q4, or the q8 kernel of fixed widths; the q8 kernel of any width
-// takes up to twice as long on wide rows.  Where the sides differ little the
-// line is not fitted: 8 x 59,815 x 768 q8 still streams, 66 / 75.
-inline bool stream_is_faster(bool q8, bool coalesced, int64_t n, int64_t d, int64_t nq) {
+// Where the sides differ little the line is not fitted: 8 x 59,815 x 768 q8
+// still streams, 65 / 78.
+inline bool stream_is_faster(bool q8, int64_t n, int64_t d, int64_t nq) {
     const bool one_pass = n <= 4096;
     double line = q8 && one_pass ? 3e8 : 5e8;
     if (one_pass && d > 512) line /= 2;
-    if (!coalesced && d > 256) line /= 2;
     return (double)nq * (double)n * (double)(d + 256) < line;
 }
 

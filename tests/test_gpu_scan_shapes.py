@@ -2,8 +2,8 @@
 that the config-shaped tests do not reach: rows of any number of 16-byte
 pieces (q8) or blocks (q4), streamed a query at a time or through the
 multi-query kernels (k past 192 always takes those with 8 or more queries),
-and the buffered selection of the streaming scans (k <= 192, past 16 on the
-fixed-width q8 rows) on tied and
+and the buffered selection of the streaming scans (k <= 192; on fixed-width q8
+rows past the lists' k) on tied and
 clustered rows.  Bar: ids and scores bit-exact with the oracle."""
 import numpy as np
 import pytest

@@ -14,8 +14,8 @@ extern "C" int rounds(int64_t tiles, int64_t nq, int64_t wgs) { return manta::ch
 extern "C" int buffered(int64_t tiles, int64_t nq, int64_t wgs, int rounds, int pitch) {
     return manta::buffered_rounds(tiles, nq, wgs, rounds, 512, pitch);
 }
-extern "C" int stream(int q8, int coalesced, int64_t n, int64_t d, int64_t nq) {
-    return manta::stream_is_faster(q8 != 0, coalesced != 0, n, d, nq);
+extern "C" int stream(int q8, int64_t n, int64_t d, int64_t nq) {
+    return manta::stream_is_faster(q8 != 0, n, d, nq);
 }
 """
 
@@ -30,7 +30,7 @@ def lib(tmp_path_factory):
     lib = C.CDLL(str(so))
     lib.rounds.argtypes = [C.c_int64, C.c_int64, C.c_int64]
     lib.buffered.argtypes = [C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int]
-    lib.stream.argtypes = [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64]
+    lib.stream.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int64]
     return lib
 
 
@@ -60,22 +60,23 @@ def test_buffered_rounds_leave_no_short_wave_of_long_parts(lib):
     assert lib.buffered(2735, 6, 256, 64, 32) == 33
 
 
-# Whole calls timed both ways, us: format, coalesced, n, d, nq, in passes, streaming.
+# Whole calls timed both ways, us: format, n, d, nq, in passes, streaming.
 TIMED = [
-    ("q8", True, 159505, 128, 8, 57, 41), ("q8", True, 23925, 384, 32, 55, 45), ("q8", True, 79753, 512, 8, 59, 50),
-    ("q8", True, 130209, 384, 32, 62, 98), ("q8", True, 79617, 1024, 8, 75, 128), ("q8", True, 11963, 1024, 32, 62, 54),
-    ("q8", True, 500, 256, 512, 39, 29), ("q8", True, 3739, 768, 128, 45, 61), ("q8", True, 1200, 768, 200, 40, 52),
-    ("q8", True, 1200, 1024, 200, 42, 61), ("q8", True, 2400, 768, 200, 44, 73), ("q8", True, 4001, 256, 64, 41, 31),
-    ("q8", False, 28089, 100, 32, 53, 44), ("q8", False, 7959, 333, 32, 52, 38), ("q8", False, 25997, 333, 32, 55, 66),
-    ("q8", False, 25475, 480, 8, 52, 45), ("q8", False, 20805, 480, 32, 57, 74), ("q8", False, 17889, 600, 32, 58, 97),
-    ("q8", False, 12191, 1000, 32, 62, 81), ("q8", False, 2099, 600, 128, 39, 65), ("q8", False, 1867, 1000, 128, 41, 63),
-    ("q8", False, 5477, 600, 32, 57, 50), ("q8", False, 16219, 900, 8, 55, 47), ("q8", False, 3047, 1000, 128, 45, 81),
-    ("q4", True, 39877, 128, 32, 57, 50), ("q4", True, 83221, 480, 8, 64, 59), ("q4", True, 49079, 992, 8, 79, 61),
-    ("q4", True, 39063, 384, 32, 62, 78), ("q4", True, 24415, 768, 32, 68, 90), ("q4", True, 3739, 768, 128, 48, 69),
-    ("q4", True, 2400, 256, 300, 74, 43), ("q4", True, 1200, 768, 300, 53, 67), ("q4", True, 1200, 1024, 300, 72, 111),
+    ("q8", 159505, 128, 8, 55, 41), ("q8", 23925, 384, 32, 56, 42), ("q8", 79753, 512, 8, 59, 50),
+    ("q8", 156251, 384, 8, 62, 99), ("q8", 78125, 1024, 8, 75, 129), ("q8", 11963, 1024, 32, 62, 52),
+    ("q8", 500, 256, 512, 37, 33), ("q8", 3739, 768, 128, 45, 52), ("q8", 1200, 768, 200, 39, 52),
+    ("q8", 1200, 1024, 200, 42, 61), ("q8", 2400, 768, 200, 44, 69), ("q8", 4001, 256, 64, 41, 31),
+    ("q8", 2400, 512, 200, 46, 59), ("q8", 1831, 384, 128, 41, 30), ("q8", 915, 1024, 128, 39, 37),
+    ("q8", 28089, 100, 32, 54, 44), ("q8", 7959, 333, 32, 54, 33), ("q8", 12203, 333, 32, 54, 37),
+    ("q8", 25475, 480, 8, 54, 43), ("q8", 11683, 600, 32, 59, 45), ("q8", 17889, 600, 32, 59, 55),
+    ("q8", 12191, 1000, 32, 62, 55), ("q8", 3047, 1000, 128, 45, 55), ("q8", 19905, 1000, 32, 63, 73),
+    ("q8", 5477, 600, 32, 58, 35), ("q8", 16219, 900, 8, 56, 37), ("q8", 3311, 900, 128, 46, 56),
+    ("q4", 39877, 128, 32, 56, 39), ("q4", 83221, 480, 8, 63, 59), ("q4", 49079, 992, 8, 79, 61),
+    ("q4", 156251, 384, 8, 69, 84), ("q4", 24415, 768, 32, 67, 90), ("q4", 3739, 768, 128, 48, 69),
+    ("q4", 2400, 256, 300, 74, 42), ("q4", 1200, 768, 300, 51, 66), ("q4", 1200, 1024, 300, 59, 97),
 ]
 
 
-@pytest.mark.parametrize("fmt,coalesced,n,d,nq,passes,stream", TIMED)
-def test_the_streaming_line_follows_the_times(lib, fmt, coalesced, n, d, nq, passes, stream):
-    assert bool(lib.stream(fmt == "q8", coalesced, n, d, nq)) == (stream < passes)
+@pytest.mark.parametrize("fmt,n,d,nq,passes,stream", TIMED)
+def test_the_streaming_line_follows_the_times(lib, fmt, n, d, nq, passes, stream):
+    assert bool(lib.stream(fmt == "q8", n, d, nq)) == (stream < passes)
