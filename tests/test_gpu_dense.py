@@ -84,3 +84,25 @@ def test_dense_scores_tile_edges(rt, n, d, nq, f16):
         rows = docs = synth.normal_f32(44, 0, n, d, 1.0)
     got = rt.dense_scores(rt.to_device(rows), rt.to_device(q)).download()
     np.testing.assert_array_equal(got, orc.dot_rows(q, docs))
+
+
+@pytest.mark.parametrize("d,nq,n", [(384, 3, 1500), (33, 17, 1500), (40, 70, 40000), (33, 30, 70001), (24, 12, 70000),
+                                    (24, 7, 70000)])
+def test_dense_nan_of_the_running_sum_stays(rt, d, nq, n):
+    """Infinities of both signs make the sum a NaN, negative on x86 and here;
+    a NaN element after that leaves its sign, as the reference's sequential
+    sum does, and positive and negative NaN rank at opposite ends."""
+    rng = np.random.default_rng(d)
+    rows = rng.standard_normal((n, d)).astype(np.float32)
+    m = rng.random((n, d)) < 3.0 / d
+    rows[m] = rng.choice(np.array([np.nan, np.inf, -np.inf, -0.0], np.float32), int(m.sum()))
+    queries = rng.standard_normal((nq, d)).astype(np.float32)
+    want = np.zeros((nq, n), np.float32)
+    with np.errstate(invalid="ignore"):
+        for c in range(d):
+            prod = queries[:, c:c + 1] * rows[None, :, c]  # (named: numpy exchanges an unnamed operand)
+            want = np.add(want, prod)
+    bits = want.view(np.uint32)
+    assert (bits == 0xFFC00000).any() and (bits == 0x7FC00000).any()
+    got = rt.dense_scores(rt.to_device(rows), rt.to_device(queries)).download()
+    np.testing.assert_array_equal(got.view(np.uint32), bits)
