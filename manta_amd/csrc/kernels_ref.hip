@@ -694,10 +694,10 @@ template <int FMT, int OP>
 static hipError_t launch_ref_scores_op(const RefArgs& a, float* out, hipStream_t s) {
     const int nq = a.set_stride ? 1 : a.nq;
     const bool few = a.n * nq < 512 * 1024;
-    // (16 queries of rows past 736 columns hold over 64 KB of LDS, one workgroup
-    // a CU: two tiles of 8 instead.  10 q4 queries x 118,304 x 1,024, dot: 334 us,
-    // now 175)
-    if (nq > 8 && !few && a.d <= 736) return launch_ref_scores_tile<FMT, OP, 4, 4, 64>(a, out, s);
+    // (16 queries of rows past 960 columns hold over half a CU's 160 KB of LDS:
+    // two tiles of 8 instead.  10 q4 queries x 118,304 x 1,024, dot: 334 us, now
+    // 175; 11 q8 queries x 546,039 x 768, cosine: 827, and 887 as two tiles)
+    if (nq > 8 && !few && a.d <= 960) return launch_ref_scores_tile<FMT, OP, 4, 4, 64>(a, out, s);
     if (nq > 4 && !few) return launch_ref_scores_tile<FMT, OP, 4, 2, 64>(a, out, s);
     // (stages of 128 columns would be half empty at the end of these rows)
     if (nq > 4 && ((a.d + 63) / 64) % 2 != 0) return launch_ref_scores_tile<FMT, OP, 8, 1, 64>(a, out, s);

@@ -60,7 +60,8 @@ def test_score_matrix_small_tiles(rt, op, fmt, d, nq, n):
 @pytest.mark.parametrize("fmt,d,nq,n", [("q8", 33, 1, 65537), ("q4", 64, 1, 40001), ("q4", 32, 2, 20000),
                                         ("q8", 1024, 5, 104861), ("q8", 100, 8, 65536), ("q4", 96, 7, 75001),
                                         ("q8", 1024, 16, 32769), ("q8", 65, 9, 58303), ("q4", 160, 19, 30001),
-                                        ("q8", 300, 1, 262147), ("q4", 1024, 9, 60001)])
+                                        ("q8", 300, 1, 262147), ("q4", 1024, 9, 60001),
+                                        ("q8", 960, 12, 43691)])
 def test_score_matrix_large_tiles(rt, op, fmt, d, nq, n):
     """Checked on the first and last rows and a stretch of the middle."""
     q = _queries(d + nq, nq, d)
